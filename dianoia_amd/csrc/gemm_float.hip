@@ -18,15 +18,33 @@
 // acc = fmadd(s, sw, acc).
 //
 // Per 32 x 32 tile and block: six v_mfma_f32_32x32x16_bf16 (three pieces x
-// two halves of the block's K) and 16 fma. A wave loads its 32 tokens'
-// fp32 x for a block (32 bytes per lane per half, straight from memory,
-// a block ahead) and splits it in registers; the weights are converted to
-// bf16 B fragments once per workgroup in LDS, with their fp32 scales.
+// two halves of the block's K, 192 clocks) and 16 fma. x is split and the
+// weights are converted to bf16 once per workgroup, on their way into LDS:
+// a wave that splits its own 32 tokens beside 64 or 128 rows spends more on
+// the VALU (about 220 instructions per block) than on the matrix cores.
 //
-// Workgroup: 256 threads, 4 waves along M (32 tokens each), SN x 32 weight
-// rows; 4-block stages double-buffered in LDS. When the tiles alone would
-// leave CUs idle, K is split over blockIdx.y and a second kernel adds the
-// partials in split order (deterministic).
+// Workgroup: 512 threads; a wave holds 64 tokens x 64 weight rows (32 x 64 in
+// the smallest tile), so a block's fragments, 16 KB of LDS reads, feed 24
+// MFMAs. Three tiles: 128 tokens x 256 rows, 64 x 256 in two block parities
+// and 32 x 128 in four (groups of waves that take the blocks of a stage in
+// turn and add their sums through LDS at the end, in order). One stage (1, 2
+// or 4 blocks) is converted into one LDS buffer while the other is
+// multiplied, its loads in flight a stage ahead. The two waves of a SIMD
+// take the two parts of a stage in opposite order, the multiplying one at
+// higher priority, so that the matrix cores and the VALU work side by side
+// (4320 x 1152 at 1024 tokens: 60 us in the same order, 48 so).
+//
+// What bounds it: the MFMAs of three pieces (25.8 GFLOP, 16 us at the 1.6
+// PFLOP/s a large bf16 product reaches here, for 4096 x 4096 at 256 tokens),
+// the conversions the matrix cores do not cover, and where K is split the
+// partials' round trip. Measured (us, graph-timed, against four waves of 32
+// tokens that each split their own x): 4096 x 4096 at 256 tokens 63.6 ->
+// 35-38, 4320 x 1152 and 1152 x 4320 at 1024 70.5 / 73.8 -> 48-52 / 47,
+// 6144 x 2048 Q4 at 512 / 64 95.9 / 28.1 -> 50-56 / 16, 1024 x 1024 at 1024
+// 24.2 -> 14.1, 8192 x 4096 at 16 48.0 -> 15.9, 3072 x 1024 at 12 11.3 -> 7.3.
+//
+// When the tiles alone would leave CUs idle, K is split over blockIdx.y and
+// a second kernel adds the partials in split order (deterministic).
 
 #include "common.h"
 #include "dnx_kernels.h"
@@ -38,11 +56,8 @@ namespace {
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
-constexpr int kThreads = 256;
-constexpr int kWaves = 4;
-constexpr int kTok = 32;        // tokens per wave (one MFMA tile of rows)
-constexpr int kBM = kWaves * kTok;
-constexpr int kKB = 4;          // blocks per stage
+constexpr int kThreads = 512;
+constexpr int kWaves = 8;
 
 struct FParams {
   const void* qs;       // Q8 int8 [rows][cols] or Q4 nibbles [rows][cols/2]
@@ -52,13 +67,17 @@ struct FParams {
   float* part;          // split partials [splits][n][rows], or null
   int rows, cols, n;
   int tiles_m, tiles;
-  int split_blocks;     // blocks per K split, a multiple of kKB
+  int split_blocks;     // blocks per K split, a multiple of the tile's parities
 };
+
+// The top halves of two dwords as one (a in the low half).
+DNX_DEV uint32_t hi16x2(uint32_t a, uint32_t b) {
+  return __builtin_amdgcn_perm(b, a, 0x07060302u);
+}
 
 // Two small integers as a pair of bf16 (exact: at most 8 significant bits).
 DNX_DEV uint32_t bf16x2(int a, int b) {
-  const uint32_t fa = __float_as_uint((float)a), fb = __float_as_uint((float)b);
-  return (fa >> 16) | (fb & 0xffff0000u);
+  return hi16x2(__float_as_uint((float)a), __float_as_uint((float)b));
 }
 
 // 8 weights of a block (k = 8c .. 8c + 7 of one K half) as one 16-byte bf16
@@ -69,208 +88,309 @@ DNX_DEV uint4 weight_frag(const int* w) {
 }
 
 // Eight floats -> the three bf16 pieces of each (p0 + p1 + p2 == x), each
-// piece as one 16-byte fragment (element j of the fragment = value j). An
-// infinity or NaN is carried whole by p0 (a quiet NaN for every NaN) with
-// zero pieces after it, so it meets the weights as the CPU's x does.
-DNX_DEV void split_frags(const float* x, uint4* p) {
+// piece as one 16-byte fragment (element j of the fragment = value j).
+// split_any: an infinity or NaN is carried whole by p0 (a quiet NaN for
+// every NaN) with zero pieces after it, so it meets the weights as the CPU's
+// x does. It is called only for the eight values that hold one.
+DNX_DEV void split_any(const float* x, uint4* p) {
   uint32_t q[3][8];
 #pragma unroll
   for (int j = 0; j < 8; j++) {
-    split3_bf16(x[j], q[0][j], q[1][j], q[2][j]);
     const uint32_t bits = __float_as_uint(x[j]);
-    if ((bits & 0x7f800000u) == 0x7f800000u) {
-      q[0][j] = (bits & 0x007fffffu) ? 0x7fc0u : bits >> 16;
-      q[1][j] = q[2][j] = 0u;
-    }
+    const float r = x[j] - __uint_as_float(bits & 0xffff0000u);
+    const uint32_t b1 = __float_as_uint(r);
+    const float r2 = r - __uint_as_float(b1 & 0xffff0000u);
+    const bool inf_nan = (bits & 0x7f800000u) == 0x7f800000u;
+    q[0][j] = inf_nan && (bits & 0x007fffffu) ? 0x7fc00000u : bits;
+    q[1][j] = inf_nan ? 0u : b1;
+    q[2][j] = inf_nan ? 0u : __float_as_uint(r2);
   }
 #pragma unroll
   for (int i = 0; i < 3; i++) {
-    p[i] = make_uint4(q[i][0] | (q[i][1] << 16), q[i][2] | (q[i][3] << 16),
-                      q[i][4] | (q[i][5] << 16), q[i][6] | (q[i][7] << 16));
+    p[i] = make_uint4(hi16x2(q[i][0], q[i][1]), hi16x2(q[i][2], q[i][3]),
+                      hi16x2(q[i][4], q[i][5]), hi16x2(q[i][6], q[i][7]));
   }
 }
 
-template <bool kQ4, int SN>
+DNX_DEV void split_frags(const float* x, uint4* p) {
+  float rest = 0.0f;   // of the first pieces: NaN when a value is infinite or NaN
+  uint32_t w[3][4];
+#pragma unroll
+  for (int j = 0; j < 8; j += 2) {
+    const uint32_t a = __float_as_uint(x[j]), b = __float_as_uint(x[j + 1]);
+    const float ra = x[j] - __uint_as_float(a & 0xffff0000u);
+    const float rb = x[j + 1] - __uint_as_float(b & 0xffff0000u);
+    const uint32_t a1 = __float_as_uint(ra), b1 = __float_as_uint(rb);
+    const float ra2 = ra - __uint_as_float(a1 & 0xffff0000u);
+    const float rb2 = rb - __uint_as_float(b1 & 0xffff0000u);
+    w[0][j / 2] = hi16x2(a, b);
+    w[1][j / 2] = hi16x2(a1, b1);
+    w[2][j / 2] = hi16x2(__float_as_uint(ra2), __float_as_uint(rb2));
+    rest += ra + rb;
+  }
+#pragma unroll
+  for (int i = 0; i < 3; i++) p[i] = make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]);
+  if (__builtin_expect(rest != rest, 0)) split_any(x, p);
+}
+
+// Shape of a workgroup's tile: WM x WN waves of TM * 32 tokens x 64 weight
+// rows, and PAR groups of them that take the blocks of a stage in turn.
+template <int WM_, int WN_, int PAR_, int TM_>
+struct Tile {
+  static constexpr int WM = WM_, WN = WN_, PAR = PAR_, TM = TM_;
+  static constexpr int BM = WM * TM * 32, BN = WN * 64;
+  static_assert(WM * WN * PAR == kWaves, "eight waves");
+  // LDS strides of one fragment row set (tokens or weight rows x 16 bytes):
+  // the pads put the four threads that write one 32-value block, and the two
+  // rows beside them, in different banks.
+  static constexpr int kFA = BM * 16 + 32, kFB = BN * 16 + 16;
+  static constexpr int kA = PAR * 12 * kFA;             // [par][piece][4 k-groups]
+  static constexpr int kB = PAR * 4 * kFB;              // [par][4 k-groups]
+  static constexpr int kStage = kA + kB + PAR * BN * 4; // + fp32 weight scales
+  static constexpr int kLds = 2 * kStage;
+  static_assert(PAR == 1 || kLds >= (PAR - 1) * BM * BN * 4, "the parities' sums reuse the stages");
+};
+
+template <bool kQ4, class T>
 __global__ void __launch_bounds__(kThreads) gemm_float_kernel(FParams p) {
-  constexpr int BN = SN * 32;
-  // LDS stage: bf16 B fragments [kb][h][khalf][row][16 B], then the fp32
-  // scales [kb][row].
-  constexpr int kFrag = kKB * 4 * BN * 16;
-  constexpr int kStage = kFrag + kKB * BN * 4;
-  constexpr int kPairs = BN * kKB;                      // (row, block) per stage
-  constexpr int PP = (kPairs + kThreads - 1) / kThreads;
-  __shared__ __align__(16) uint8_t lds[2 * kStage];
+  constexpr int WM = T::WM, WN = T::WN, PAR = T::PAR, TM = T::TM, BM = T::BM, BN = T::BN;
+  constexpr int UA = BM * 4 * PAR, PA = (UA + kThreads - 1) / kThreads;   // 8 x values each
+  constexpr int UB = BN * 2 * PAR, PB = (UB + kThreads - 1) / kThreads;   // 16 weights each
+  constexpr int US = BN * PAR, PS = (US + kThreads - 1) / kThreads;       // weight scales
+  __shared__ __align__(16) uint8_t lds[T::kLds];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int par = wave / (WM * WN), wm = wave % (WM * WN) / WN, wn = wave % WN;
   const int K = p.cols, B = K / kBlock, M = p.n, N = p.rows;
   // XCD-aware order (workgroups are dealt round-robin to the 8 XCDs): each
   // XCD walks a contiguous run of tiles, all token tiles of its weight rows.
-  const int i = blockIdx.x;
-  const int t = (p.tiles % 8 == 0) ? (i % 8) * (p.tiles / 8) + i / 8 : i;
-  const int tm = t % p.tiles_m, tn = t / p.tiles_m;
-  const int n0 = tn * BN;
-  const int m0 = tm * kBM + wave * kTok;
+  const int i0 = blockIdx.x;
+  const int t = (p.tiles % 8 == 0) ? (i0 % 8) * (p.tiles / 8) + i0 / 8 : i0;
+  const int m0 = t % p.tiles_m * BM, n0 = t / p.tiles_m * BN;
   const int b_begin = blockIdx.y * p.split_blocks;
-  const int b_end = min(B, b_begin + p.split_blocks);
-  const int stages = (b_end - b_begin + kKB - 1) / kKB;
+  const int nb = min(B, b_begin + p.split_blocks) - b_begin;   // this split's blocks
+  const int steps = (nb + PAR - 1) / PAR;
 
-  const int wbytes = kQ4 ? 16 : 32;
+  constexpr int wbytes = kQ4 ? 16 : 32, sbytes = kQ4 ? 2 : 4;
+  constexpr int kFar = -(1 << 20);   // past every operand: reads zeros
   const i32x4 rq = buffer_rsrc(p.qs, (uint32_t)((size_t)N * B * wbytes));
-  const i32x4 rs = buffer_rsrc(p.scales, (uint32_t)((size_t)N * B * (kQ4 ? 2 : 4)));
+  const i32x4 rs = buffer_rsrc(p.scales, (uint32_t)((size_t)N * B * sbytes));
   const i32x4 rx = buffer_rsrc(p.x, (uint32_t)((size_t)M * K * 4));
 
-  // ---- weight staging: thread q takes (row q / kKB, block q % kKB)
-  i32x4 wq[PP][2];
-  int ws[PP];
-  auto load_w = [&](int s) {
-    const int b0 = b_begin + s * kKB;
+  // ---- staging: what each thread carries from memory to LDS in a step.
+  // x: (token, block, group of 8 values), four threads to a token's 128-byte
+  // block; weights: (row, block, half of 16 values); scales: (row, block).
+  i32x4 xr[PA][2], wr[PB];
+  int sr[PS];
+  auto load_step = [&](int s) {
+    const int b0 = b_begin + s * PAR, left = nb - s * PAR;   // blocks from b0 on
 #pragma unroll
-    for (int e = 0; e < PP; e++) {
-      const int q = e * kThreads + tid;
-      const int row = q / kKB, b = b0 + q % kKB;
-      const bool ok = q < kPairs && n0 + row < N && b < b_end;
-      const int off = ok ? ((n0 + row) * B + b) * wbytes : -(1 << 20);
-      wq[e][0] = dnx_raw_buffer_load_v4i32(rq, off, 0, 0);
-      if (!kQ4) wq[e][1] = dnx_raw_buffer_load_v4i32(rq, off + 16, 0, 0);
-      ws[e] = kQ4 ? (int)(uint16_t)dnx_raw_buffer_load_i16(rs, ok ? ((n0 + row) * B + b) * 2 : -4, 0, 0)
-                  : dnx_raw_buffer_load_i32(rs, ok ? ((n0 + row) * B + b) * 4 : -4, 0, 0);
+    for (int e = 0; e < PA; e++) {
+      const int u = e * kThreads + tid, f = u & 3, tok = (u >> 2) % BM, blk = (u >> 2) / BM;
+      const bool ok = u < UA && m0 + tok < M && blk < left;
+      const int off = ok ? ((m0 + tok) * K + (b0 + blk) * kBlock + 8 * f) * 4 : kFar;
+      xr[e][0] = dnx_raw_buffer_load_v4i32(rx, off, 0, 0);
+      xr[e][1] = dnx_raw_buffer_load_v4i32(rx, off + 16, 0, 0);
+    }
+#pragma unroll
+    for (int e = 0; e < PB; e++) {
+      const int u = e * kThreads + tid, h = u & 1, blk = (u >> 1) % PAR, row = u / (2 * PAR);
+      const bool ok = u < UB && n0 + row < N && blk < left;
+      // A Q4 block's 16 bytes hold both halves (low and high nibbles).
+      const int off = ((n0 + row) * B + b0 + blk) * wbytes + (kQ4 ? 0 : 16 * h);
+      wr[e] = dnx_raw_buffer_load_v4i32(rq, ok ? off : kFar, 0, 0);
+    }
+#pragma unroll
+    for (int e = 0; e < PS; e++) {
+      const int u = e * kThreads + tid, blk = u % PAR, row = u / PAR;
+      const bool ok = u < US && n0 + row < N && blk < left;
+      const int off = ok ? ((n0 + row) * B + b0 + blk) * sbytes : kFar;
+      // Q4: the raw 16 bits (an operation on them here would wait for them).
+      sr[e] = kQ4 ? (int)dnx_raw_buffer_load_i16(rs, off, 0, 0)
+                  : dnx_raw_buffer_load_i32(rs, off, 0, 0);
     }
   };
-  auto store_w = [&](int buf) {
-    uint8_t* base = lds + buf * kStage;
+  auto store_step = [&](int buf) {
+    uint8_t* base = lds + buf * T::kStage;
 #pragma unroll
-    for (int e = 0; e < PP; e++) {
-      const int q = e * kThreads + tid;
-      if (q >= kPairs) continue;
-      const int row = q / kKB, kb = q % kKB;
-      int w[32];
-      if (kQ4) {
-        const uint32_t v[4] = {(uint32_t)wq[e][0].x, (uint32_t)wq[e][0].y, (uint32_t)wq[e][0].z,
-                               (uint32_t)wq[e][0].w};
+    for (int e = 0; e < PA; e++) {
+      const int u = e * kThreads + tid, f = u & 3, tok = (u >> 2) % BM, blk = (u >> 2) / BM;
+      if (UA % kThreads != 0 && u >= UA) break;
+      float xv[8];
 #pragma unroll
-        for (int k = 0; k < 16; k++) {
-          const uint32_t byte = (v[k >> 2] >> (8 * (k & 3))) & 0xffu;
-          w[k] = (int)(byte & 15u) - 8;
-          w[k + 16] = (int)(byte >> 4) - 8;
-        }
-      } else {
-        const uint32_t v[8] = {(uint32_t)wq[e][0].x, (uint32_t)wq[e][0].y, (uint32_t)wq[e][0].z,
-                               (uint32_t)wq[e][0].w, (uint32_t)wq[e][1].x, (uint32_t)wq[e][1].y,
-                               (uint32_t)wq[e][1].z, (uint32_t)wq[e][1].w};
-#pragma unroll
-        for (int k = 0; k < 32; k++) w[k] = (int)(int8_t)(v[k >> 2] >> (8 * (k & 3)));
+      for (int j = 0; j < 4; j++) {
+        xv[j] = __int_as_float(xr[e][0][j]);
+        xv[4 + j] = __int_as_float(xr[e][1][j]);
       }
-      // Fragment (h, c) holds k = 16 h + 8 c .. + 7.
+      uint4 q[3];
+      split_frags(xv, q);
 #pragma unroll
-      for (int f = 0; f < 4; f++) {
-        *(uint4*)(base + ((kb * 4 + f) * BN + row) * 16) = weight_frag(w + 8 * f);
+      for (int pc = 0; pc < 3; pc++)
+        *(uint4*)(base + ((blk * 3 + pc) * 4 + f) * T::kFA + tok * 16) = q[pc];
+    }
+#pragma unroll
+    for (int e = 0; e < PB; e++) {
+      const int u = e * kThreads + tid, h = u & 1, blk = (u >> 1) % PAR, row = u / (2 * PAR);
+      if (UB % kThreads != 0 && u >= UB) break;
+      int w[16];
+#pragma unroll
+      for (int k = 0; k < 16; k++) {
+        const uint32_t v = (uint32_t)wr[e][k >> 2];
+        w[k] = kQ4 ? (int)((v >> (8 * (k & 3) + 4 * h)) & 15u) - 8
+                   : (int)(int8_t)(v >> (8 * (k & 3)));
       }
-      const float sw = kQ4 ? half_bits_to_float((uint16_t)ws[e]) : __int_as_float(ws[e]);
-      *(float*)(base + kFrag + (kb * BN + row) * 4) = sw;
+      uint8_t* d = base + T::kA + (blk * 4 + 2 * h) * T::kFB + row * 16;
+      *(uint4*)d = weight_frag(w);
+      *(uint4*)(d + T::kFB) = weight_frag(w + 8);
+    }
+#pragma unroll
+    for (int e = 0; e < PS; e++) {
+      const int u = e * kThreads + tid, blk = u % PAR, row = u / PAR;
+      if (US % kThreads != 0 && u >= US) break;
+      const float sw = kQ4 ? half_bits_to_float((uint16_t)sr[e]) : __int_as_float(sr[e]);
+      *(float*)(base + T::kA + T::kB + (blk * BN + row) * 4) = sw;
     }
   };
 
-  // ---- this wave's x: lane l holds token m0 + l % 32, k = 8 (l / 32) + 0..7
-  // of each K half (16 h); tokens past n read zeros.
-  const int xm = m0 + (lane & 31);
-  auto load_x = [&](int b, i32x4* xr) {
-    const bool ok = xm < M && b < b_end;
+  v16f acc[TM][2];
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const int off = ok ? (xm * K + b * kBlock + 16 * h + 8 * (lane >> 5)) * 4 : -(1 << 20);
-      xr[2 * h] = dnx_raw_buffer_load_v4i32(rx, off, 0, 0);
-      xr[2 * h + 1] = dnx_raw_buffer_load_v4i32(rx, off + 16, 0, 0);
-    }
-  };
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int v = 0; v < 16; v++) acc[i][j][v] = 0.0f;
 
-  v16f acc[SN];
-#pragma unroll
-  for (int j = 0; j < SN; j++)
-#pragma unroll
-    for (int v = 0; v < 16; v++) acc[j][v] = 0.0f;
-
-  i32x4 xcur[4], xnext[4];
-  load_x(b_begin, xcur);
-  load_w(0);
-  store_w(0);
+  const int l32 = lane & 31, c = lane >> 5;
+  load_step(0);
+  store_step(0);
+  if (steps > 1) load_step(1);
   __syncthreads();
-  for (int s = 0; s < stages; s++) {
-    const int buf = s & 1;
-    if (s + 1 < stages) load_w(s + 1);
-    const uint8_t* base = lds + buf * kStage;
-    const int b0 = b_begin + s * kKB;
-#pragma unroll 1
-    for (int kb = 0; kb < kKB; kb++) {
-      load_x(b0 + kb + 1, xnext);
-      // The three bf16 pieces of this lane's 16 x values, per K half.
-      uint4 a[2][3];
+  // The two waves of a SIMD (waves w and w + 4) take a step's parts in
+  // opposite order, so that one's matrix work runs beside the other's
+  // conversions: in the same order both wait for the same unit at once.
+  const bool stage_first = wave < kWaves / 2;
+  auto stage_next = [&](int s) {
+    if (s + 1 < steps) {
+      store_step((s + 1) & 1);
+      if (s + 2 < steps) load_step(s + 2);
+    }
+  };
+  for (int s = 0; s < steps; s++) {
+    const uint8_t* base = lds + (s & 1) * T::kStage;
+    if (stage_first) stage_next(s);
+    if (s * PAR + par < nb) {   // the wave's block of this stage exists
+      const uint8_t* ab = base + par * 12 * T::kFA + (wm * TM * 32 + l32) * 16;
+      const uint8_t* bb = base + T::kA + par * 4 * T::kFB + (wn * 64 + l32) * 16;
+      __builtin_amdgcn_s_setprio(1);   // before the other wave's conversions
+      v16f d[TM][2];
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+          for (int v = 0; v < 16; v++) d[i][j][v] = 0.0f;
 #pragma unroll
       for (int h = 0; h < 2; h++) {
-        float xv[8];
+        bf8 a[TM][3], w[2];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-          xv[j] = __int_as_float(xcur[2 * h][j]);
-          xv[4 + j] = __int_as_float(xcur[2 * h + 1][j]);
-        }
-        split_frags(xv, a[h]);
-      }
-      // The SN tiles' MFMAs interleaved (independent accumulators), then
-      // one fma per output with the row's scale.
-      v16f d[SN];
+        for (int j = 0; j < 2; j++)
+          w[j] = __builtin_bit_cast(bf8, *(const uint4*)(bb + (2 * h + c) * T::kFB + j * 512));
 #pragma unroll
-      for (int j = 0; j < SN; j++)
+        for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int v = 0; v < 16; v++) d[j][v] = 0.0f;
-#pragma unroll
-      for (int h = 0; h < 2; h++) {
-        bf8 bw[SN];
-#pragma unroll
-        for (int j = 0; j < SN; j++) {
-          const int row = j * 32 + (lane & 31);
-          bw[j] = __builtin_bit_cast(
-              bf8, *(const uint4*)(base + ((kb * 4 + 2 * h + (lane >> 5)) * BN + row) * 16));
-        }
+          for (int pc = 0; pc < 3; pc++)
+            a[i][pc] = __builtin_bit_cast(
+                bf8, *(const uint4*)(ab + (pc * 4 + 2 * h + c) * T::kFA + i * 512));
 #pragma unroll
         for (int pc = 0; pc < 3; pc++)
 #pragma unroll
-          for (int j = 0; j < SN; j++) {
-            d[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8, a[h][pc]),
-                                                           bw[j], d[j], 0, 0, 0);
-          }
+          for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+              d[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][pc], w[j], d[i][j], 0, 0, 0);
       }
 #pragma unroll
-      for (int j = 0; j < SN; j++) {
-        const float sw = *(const float*)(base + kFrag + (kb * BN + j * 32 + (lane & 31)) * 4);
+      for (int j = 0; j < 2; j++) {
+        const float sw =
+            *(const float*)(base + T::kA + T::kB + (par * BN + wn * 64 + j * 32 + l32) * 4);
 #pragma unroll
-        for (int v = 0; v < 16; v++) acc[j][v] = fmaf(d[j][v], sw, acc[j][v]);
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int v = 0; v < 16; v++) acc[i][j][v] = fmaf(d[i][j][v], sw, acc[i][j][v]);
       }
-#pragma unroll
-      for (int r = 0; r < 4; r++) xcur[r] = xnext[r];
+      __builtin_amdgcn_s_setprio(0);
     }
-    if (s + 1 < stages) store_w(buf ^ 1);
+    if (!stage_first) stage_next(s);
     __syncthreads();
   }
 
-  float* out = p.part ? p.part + (size_t)blockIdx.y * M * N : p.y;
+  // The parities' sums, added in parity order by parity 0's waves.
+  if constexpr (PAR > 1) {
+    float* red = (float*)lds + wave % (WM * WN) * (TM * 2 * 16 * 64) + lane;
 #pragma unroll
-  for (int j = 0; j < SN; j++) {
-    const int r = n0 + j * 32 + (lane & 31);
-    if (r >= N) continue;
+    for (int q = 1; q < PAR; q++) {
+      float* mine = red + (q - 1) * BM * BN;
+      if (par == q) {
 #pragma unroll
-    for (int v = 0; v < 16; v++) {
-      const int m = m0 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);
-      if (m < M) store_wt(out + (size_t)m * N + r, acc[j][v]);
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) mine[((i * 2 + j) * 16 + v) * 64] = acc[i][j][v];
+      }
+    }
+    __syncthreads();
+    if (par != 0) return;
+#pragma unroll
+    for (int q = 1; q < PAR; q++) {
+      const float* theirs = red + (q - 1) * BM * BN;
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+          for (int v = 0; v < 16; v++) acc[i][j][v] += theirs[((i * 2 + j) * 16 + v) * 64];
     }
   }
+  float* out = p.part ? p.part + (size_t)blockIdx.y * M * N : p.y;
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const int r = n0 + wn * 64 + j * 32 + l32;
+      if (r >= N) continue;
+#pragma unroll
+      for (int v = 0; v < 16; v++) {
+        const int m = m0 + (wm * TM + i) * 32 + (v >> 2) * 8 + c * 4 + (v & 3);
+        if (m < M) store_wt(out + (size_t)m * N + r, acc[i][j][v]);
+      }
+    }
 }
 
-// y = the split partials summed in split order (deterministic).
-__global__ void __launch_bounds__(kThreads) float_splitk_reduce_kernel(
+// y = the split partials summed in split order (deterministic), four
+// outputs to a thread where they are whole 16-byte pieces.
+template <bool kVec>
+__global__ void __launch_bounds__(256) float_splitk_reduce_kernel(
     const float* __restrict__ part, float* __restrict__ y, int64_t count, int splits) {
-  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < count;
-       i += (int64_t)gridDim.x * kThreads) {
-    store_wt(y + i, split_sum(part, count, i, splits));
+  const int64_t items = kVec ? count / 4 : count;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < items;
+       i += (int64_t)gridDim.x * 256) {
+    if constexpr (kVec) {
+      f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+      for (int z0 = 0; z0 < splits; z0 += 4) {   // four splits' loads together
+        f32x4 t[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          t[u] = ((const f32x4*)part)[(size_t)min(z0 + u, splits - 1) * items + i];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          if (z0 + u < splits) v = z0 + u == 0 ? t[u] : v + t[u];
+      }
+      store_wt4(y + 4 * i, make_float4(v.x, v.y, v.z, v.w));
+    } else {
+      store_wt(y + i, split_sum(part, count, i, splits));
+    }
   }
 }
 
@@ -295,10 +415,9 @@ float* part_workspace(size_t bytes) {
   return gPart;
 }
 
-template <bool kQ4, int SN>
+template <bool kQ4, class T>
 int launch(const void* qs, const void* scales, const float* x, float* y, int64_t rows,
-           int64_t cols, int64_t n, hipStream_t stream) {
-  constexpr int BN = SN * 32;
+           int64_t cols, int64_t n, int splits, hipStream_t stream) {
   FParams p{};
   p.qs = qs;
   p.scales = scales;
@@ -307,14 +426,11 @@ int launch(const void* qs, const void* scales, const float* x, float* y, int64_t
   p.rows = (int)rows;
   p.cols = (int)cols;
   p.n = (int)n;
-  p.tiles_m = (int)((n + kBM - 1) / kBM);
-  p.tiles = p.tiles_m * (int)((rows + BN - 1) / BN);
+  p.tiles_m = (int)((n + T::BM - 1) / T::BM);
+  p.tiles = p.tiles_m * (int)((rows + T::BN - 1) / T::BN);
   const int B = (int)(cols / kBlock);
-  const int max_splits = (B + kKB - 1) / kKB;
-  int splits = 1;
-  if (p.tiles < 256) splits = min((512 + p.tiles - 1) / p.tiles, max_splits);
   p.split_blocks = (B + splits - 1) / splits;
-  p.split_blocks = (p.split_blocks + kKB - 1) / kKB * kKB;
+  p.split_blocks = (p.split_blocks + T::PAR - 1) / T::PAR * T::PAR;
   splits = (B + p.split_blocks - 1) / p.split_blocks;
   const int64_t count = n * rows;
   p.part = nullptr;
@@ -322,16 +438,48 @@ int launch(const void* qs, const void* scales, const float* x, float* y, int64_t
     p.part = part_workspace((size_t)splits * count * 4);
     if (p.part == nullptr) return DNX_ENOMEM;
   }
-  hipLaunchKernelGGL((gemm_float_kernel<kQ4, SN>), dim3((unsigned)p.tiles, (unsigned)splits),
+  hipLaunchKernelGGL((gemm_float_kernel<kQ4, T>), dim3((unsigned)p.tiles, (unsigned)splits),
                      dim3(kThreads), 0, stream, p);
   if (hipGetLastError() != hipSuccess) return DNX_ELAUNCH;
   if (splits > 1) {
-    const int64_t blocks = (count + kThreads - 1) / kThreads;
-    hipLaunchKernelGGL(float_splitk_reduce_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)),
-                       dim3(kThreads), 0, stream, p.part, y, count, splits);
+    const bool vec = count % 4 == 0 && ((uintptr_t)y & 15) == 0;
+    const int64_t blocks = ((vec ? count / 4 : count) + 255) / 256;
+    hipLaunchKernelGGL(vec ? float_splitk_reduce_kernel<true> : float_splitk_reduce_kernel<false>,
+                       dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream,
+                       p.part, y, count, splits);
     if (hipGetLastError() != hipSuccess) return DNX_ELAUNCH;
   }
   return DNX_OK;
+}
+
+// What a tile and K split cost, in us: rounds of 256 workgroups (a tile's
+// LDS holds a CU to one) times a fixed part and the stages of a split, and
+// the partials' round trip. The constants are a fit to 1500 runs (40 shapes
+// of 512..8192 rows, 512..4096 columns, 5..1024 tokens, Q4 and Q8): it picks
+// within 1% of the fastest of them on average, 8% at worst.
+struct FloatCost {
+  double us;
+  int splits;
+};
+
+template <class T>
+FloatCost float_cost(int64_t rows, int64_t cols, int64_t n, double round_us, double stage_us,
+                     bool may_split) {
+  const int64_t tiles = ((n + T::BM - 1) / T::BM) * ((rows + T::BN - 1) / T::BN);
+  const int64_t B = cols / kBlock;
+  FloatCost best{1e30, 1};
+  for (int want : {1, 2, 3, 4, 6, 8, 12, 16}) {
+    if (want > B || (want > 1 && !may_split)) break;
+    const int64_t run = ((B + want - 1) / want + T::PAR - 1) / T::PAR * T::PAR;
+    const int64_t splits = (B + run - 1) / run;
+    // Partials of more than 1 GiB are not worth their memory.
+    if (splits > 1 && splits * n * rows > (1ll << 28)) break;
+    const double rounds = (double)((tiles * splits + 255) / 256);
+    const double us = rounds * (round_us + stage_us * (double)(run / T::PAR)) +
+                      (splits > 1 ? 1.8 + 1.5e-6 * (double)(splits * n * rows) : 0.0);
+    if (us < best.us) best = {us, want};
+  }
+  return best;
 }
 
 template <bool kQ4>
@@ -347,10 +495,21 @@ int launch_float(const void* qs, const void* scales, const float* x, float* y, i
       ((uintptr_t)scales & (kQ4 ? 1 : 3))) {
     return DNX_EINVAL;
   }
-  // 128 weight rows per workgroup while that keeps the CUs busy, else 64.
-  const int64_t tiles128 = ((n + kBM - 1) / kBM) * ((rows + 127) / 128);
-  if (tiles128 >= 256) return launch<kQ4, 4>(qs, scales, x, y, rows, cols, n, stream);
-  return launch<kQ4, 2>(qs, scales, x, y, rows, cols, n, stream);
+  // The tile and K split the measured costs put lowest. With 256 tiles of
+  // 128 tokens x 64 rows or more K stays whole: such calls need no memory of
+  // the library's own (a split would gain at most 9% on them).
+  const bool may_split = ((n + 127) / 128) * ((rows + 63) / 64) < 256;
+  const FloatCost costs[] = {float_cost<Tile<2, 4, 1, 2>>(rows, cols, n, 3.1, 1.13, may_split),
+                             float_cost<Tile<1, 4, 2, 2>>(rows, cols, n, 3.4, 1.28, may_split),
+                             float_cost<Tile<1, 2, 4, 1>>(rows, cols, n, 2.4, 1.01, may_split)};
+  const FloatCost& a = costs[0];
+  const FloatCost& b = costs[1];
+  const FloatCost& c = costs[2];
+  if (c.us <= a.us && c.us <= b.us)
+    return launch<kQ4, Tile<1, 2, 4, 1>>(qs, scales, x, y, rows, cols, n, c.splits, stream);
+  if (b.us <= a.us)
+    return launch<kQ4, Tile<1, 4, 2, 2>>(qs, scales, x, y, rows, cols, n, b.splits, stream);
+  return launch<kQ4, Tile<2, 4, 1, 2>>(qs, scales, x, y, rows, cols, n, a.splits, stream);
 }
 
 }  // namespace

@@ -73,6 +73,38 @@ def test_float_gemm_within_tolerance(gpu_ready, orc, fmt, rows, cols, n):
     assert np.all(np.abs(y - ref) <= 1e-4 + 1e-5 * np.abs(ref))
 
 
+# The edges of the tiles (32, 64 and 128 tokens; 128 and 256 rows), block
+# counts that leave a stage of 1, 2 or 4 blocks unfilled, and shapes that take
+# each of the three tiles, whole and with K split. The bar is the one above:
+# the products are exact, and float32 sums of K terms stay below
+# K * 2^-24 sum|terms| = 1.6e-4 at most and near sqrt(K) * 2^-24 in fact.
+@pytest.mark.parametrize("fmt", ["q8", "q4"])
+@pytest.mark.parametrize("rows,cols,n", [(127, 32, 31), (128, 64, 32), (129, 96, 33), (255, 160, 63),
+                                         (256, 224, 64), (257, 288, 65), (640, 1056, 127),
+                                         (385, 544, 129), (2912, 1056, 472), (3539, 352, 805),
+                                         (4320, 1152, 257)])
+def test_float_gemm_tile_edges(gpu_ready, fmt, rows, cols, n):
+    print(f"float gemm edges {fmt} {rows}x{cols} n={n}", flush=True)
+    rng = np.random.default_rng(rows + 3 * cols + n)
+    qs, sc = (synth.q8_weights if fmt == "q8" else synth.q4_weights)(rng, rows, cols)
+    xs = synth.activations(rng, n, cols)
+    xs[n // 2, cols // 2] = np.inf   # whole in one piece: no NaN beside it
+    xs[n - 1, cols - 1] = -2e36      # 2e36 * 127 is still a float32 (as on the CPU, past it not)
+    y = gemm_float(fmt, qs, sc, xs, rows, cols, n)
+    finite = np.delete(np.arange(n), n // 2)
+    exact, mag = exact_mode0(fmt, qs, sc, xs[finite])
+    assert np.max(np.abs(y[finite] - exact) / np.maximum(mag, 1e-30)) < 1e-5
+    if fmt == "q8":
+        w = qs[:, cols // 2].astype(np.float64) * sc[:, cols // 64]
+    else:
+        b, k = divmod(cols // 2, 32)
+        byte = qs[:, b * 16 + k % 16]
+        w = ((byte & 15 if k < 16 else byte >> 4).astype(np.float64) - 8) * sc.view(np.float16)[:, b]
+    assert np.array_equal(np.isposinf(y[n // 2]), w > 0)
+    assert np.array_equal(np.isneginf(y[n // 2]), w < 0)
+    assert np.array_equal(np.isnan(y[n // 2]), w == 0)
+
+
 def test_float_gemm_reference_gpu_test_shapes(gpu_ready, orc):
     """The reference's own GPU linear test (test/gpu_linear_test.dart:26-45):
     weights and inputs uniform in [-1, 1), within 1e-4 + 1e-5 |cpu| of CPU
