@@ -12,6 +12,7 @@
 // Built with -ffp-contract=off: no multiply-add is fused unless written as
 // fmaf.
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -792,28 +793,76 @@ attention_combine_kernel(const float* __restrict__ ws, const float* __restrict__
   }
 }
 
-// Attention of many tokens (prefill) on the fp32 matrix cores. A wave
-// takes 16 queries of one head, a workgroup 4 waves sharing one KV head
-// (GW heads of a GQA group x 4 / GW query blocks), and the workgroup walks
-// its keys in tiles of 32 staged in LDS (K row-major, V transposed), so a
-// tile is read once for up to 64 queries. Per tile and wave:
-// * S^T = K Q^T on v_mfma_f32_16x16x4f32: A = 16 keys x 4 dims (K from LDS,
-//   dims g * hd / 4 + s for lane group g), B = 4 dims x 16 queries (Q held
-//   in registers); a lane ends with 8 scores of its query (column), so the
-//   online softmax needs two cross-lane exchanges per tile;
-// * O^T += V^T P^T: the lane's exponentials are already the B operand of
-//   step s (keys (s / 4) * 16 + 4 g + s % 4), V^T tiles come from LDS.
-// The running (max, sum) rescale O when the max grows (flash attention).
+// Attention of many tokens (prefill) on the bf16 matrix cores, float32 in and
+// out. Every float32 operand is the exact sum of three bf16 pieces (8
+// significant bits each); of the nine piece products of a q.k or p.v term the
+// six with i + j <= 2 are formed, the others lie below 2^-23 of the term, and
+// the sums are float32. Six bf16 MFMAs cost less than half of the float32
+// ones they replace (v_mfma_f32_16x16x4f32: 32 multiply-adds a clock and
+// SIMD, 16x16x32_bf16: 512).
+//
+// A wave takes 16 queries of one head, a workgroup 4 waves sharing one KV
+// head (GW heads of a GQA group x 4 / GW query blocks); it walks its keys in
+// tiles of KT, split into their pieces once per workgroup on the way into
+// LDS (the next tile's values are in registers meanwhile). Per tile and wave:
+// * S^T = K Q^T: A = 16 keys x 32 dims (LDS), B = 32 dims x 16 queries (the
+//   pieces of Q, held in registers); lane l ends with the scores of query
+//   l % 16 for keys 4 (l / 16) + 0..3 of each 16, so the online softmax
+//   needs two lane exchanges for the max and two for the sum;
+// * O^T += V^T P^T: the lane's probabilities, split in registers, are the B
+//   operand as they are if k slot j of lane group g stands for key 4 g + j
+//   (j < 4) or 16 + 4 g + j - 4; V^T is staged in that order.
+// A tile's products start from zero and join the running sums in one
+// multiply-add, so a long run rounds once a tile (64 bits say 3.9e-7 after
+// 4000 keys where sums carried through the MFMAs had 9.5e-7).
+// A wave whose queries see no key of a tile skips it; only tiles at the edge
+// of the causal or window range are masked. A wave that meets an
+// infinity or NaN (in Q, or in a tile that it works on) forms its rows anew
+// in plain float32 from memory at the end (slow, and rare).
+//
 // With `splits` > 1 a workgroup takes a run of tiles_per_split tiles and
 // writes per (token, head) the partial (m, l, o) rows that
-// attention_combine_kernel adds (for long contexts with few query blocks);
-// otherwise it writes the output, gated. fp32 throughout: the sums run in
-// another order than the oracle's, and the softmax exponentials use the
-// hardware exp2 (__expf, a few ulp) instead of expf.
+// attention_combine_rows_kernel adds; one whose run lies past its queries'
+// keys writes nothing (live_splits). Otherwise it writes the output, gated.
+// m is in units of log2: exponentials use the hardware exp2 of a fused
+// multiply-add, one rounding before it.
+//
+// What bounds it: at prompt chunks the latency of one pass (launch, first
+// loads, splitting, two barriers: about 8 us with one tile, 1.8 us for each
+// more), at long prompts the MFMAs (six times the product's 2 flops, 215 of
+// 400 us at the 1.6 PFLOP/s a large bf16 product reaches) and the splitting
+// and softmax they do not cover. Measured with the combine (us, graph-timed,
+// against the float32 MFMAs; heads / KV heads, hd): 64 tokens after 256,
+// 16 / 8, 128: 14.7 -> 11.9; 37 after 500, 8 / 8, 64: 11.3 -> 8.2; 512 from
+// 0, 32 / 8, 128: 42.7 -> 33.7; 1000 after 1000, 16 / 8, 128: 169 -> 98;
+// 1024 after 4000, 8 / 4, 64: 122 -> 80. 32 queries a wave (32x32x16 MFMAs,
+// half the LDS reads) gained 8% on the longest but needed 256 registers, and
+// took 13.2 us where this takes 9.1 for one tile.
 constexpr int kPQ = 16;   // queries per wave
-constexpr int kPK = 32;   // keys per tile
 
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+
+template <int HD>
+struct PrefillTile {
+  static constexpr int KT = 4096 / HD;          // keys per tile: 32 or 64
+  static constexpr int KS = KT * 16 + 16;       // K: one 8-dim group of all keys, + pad
+  static constexpr int VS = HD * 16;            // V^T: 8 keys of all dims
+  static constexpr int kK = 3 * (HD / 8) * KS;  // [piece][dim group][key][16 B]
+  static constexpr int kV = 3 * (KT / 8) * VS;  // [piece][key group][dim][16 B]
+};
+
+// The tiles of a workgroup's queries (tokens first .. last): the range of
+// its keys, and how many splits of tps tiles they fill.
+struct KeyRange {
+  int start, end;
+};
+DNX_DEV KeyRange key_range(int position, int first, int last, int window) {
+  return {window > 0 ? max(0, position + first - window + 1) : 0, position + last + 1};
+}
+DNX_DEV int live_splits(KeyRange r, int kt, int tps) {
+  return ((r.end - r.start + kt - 1) / kt + tps - 1) / tps;
+}
 
 // Max / sum over lanes i, i ^ 16, i ^ 32 and i ^ 48 (lane i % 16 of the four
 // 16-lane rows), every lane getting the result, on gfx950's VALU lane swaps:
@@ -837,263 +886,404 @@ DNX_DEV float rows4_sum(float v) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// Eight floats as three bf16 fragments (piece i of value j in element j),
+// each piece the rest rounded to nearest: the terms that are not formed are
+// then as often too small as too large. Returns a finite number, or an
+// infinity or NaN if a value is one (or rounds to one as bf16).
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+DNX_DEV float split_pieces(const float* x, uint4* p) {
+  float rest = 0.0f;
+  uint32_t w[3][4];
+#pragma unroll
+  for (int j = 0; j < 8; j += 2) {
+    f32x2 v = {x[j], x[j + 1]};
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      w[i][j / 2] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf2));
+      if (i == 2) break;
+      v.x -= __uint_as_float(w[i][j / 2] << 16);
+      v.y -= __uint_as_float(w[i][j / 2] & 0xffff0000u);
+      if (i == 0) rest += v.x + v.y;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 3; i++) p[i] = make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]);
+  return rest;
+}
+
+// acc += A B over the six piece products, the smallest first.
+DNX_DEV v4f mfma_pieces(const uint4* a, const uint4* b, v4f acc) {
+  constexpr int kA[6] = {2, 1, 0, 1, 0, 0}, kB[6] = {0, 1, 2, 0, 1, 0};
+#pragma unroll
+  for (int i = 0; i < 6; i++)
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, a[kA[i]]),
+                                                  __builtin_bit_cast(bf8, b[kB[i]]), acc, 0, 0, 0);
+  return acc;
+}
+
+// The rows of a wave's queries over keys k_lo .. k_hi - 1 in plain float32,
+// for operands that have no pieces (infinities, NaN): a query at a time, a
+// lane to a key for the scores and to HD / 64 dims for the values. Hidden
+// keys count for nothing, whatever they hold.
+template <int HD>
+DNX_DEV void prefill_plain(
+    const float* q, const float* keys, const float* values, const float* gate, float* out,
+    float* ws, int position, int n, int heads, int head, int kv_dim, int window, float sl, int t0,
+    int k_lo, int k_hi, int splits, int split, int lane) {
+  constexpr int ND = HD / 64;
+#pragma unroll 1
+  for (int tok = t0; tok < min(t0 + kPQ, n); tok++) {
+    const int qpos = position + tok;
+    const size_t th = (size_t)tok * heads + head;
+    const float* qp = q + th * HD;
+    const int lo = window > 0 ? max(k_lo, qpos - window + 1) : k_lo, hi = min(k_hi, qpos + 1);
+    float m = -INFINITY, l = 0.0f, o[ND] = {};
+#pragma unroll 1
+    for (int k0 = lo; k0 < hi; k0 += 64) {
+      const bool live = k0 + lane < hi;
+      const float* k = keys + (size_t)(live ? k0 + lane : lo) * kv_dim;
+      float s = 0.0f;
+#pragma unroll 1
+      for (int e = 0; e < HD; e++) s = fmaf(k[e], qp[e], s);
+      s = live ? s : -INFINITY;
+      const float m_new = fmaxf(m, wave_max(s) * sl), ref = m_new == -INFINITY ? 0.0f : m_new;
+      const float p = live ? __builtin_amdgcn_exp2f(fmaf(s, sl, -ref)) : 0.0f;
+      const float alpha = __builtin_amdgcn_exp2f(m - ref);
+      l = l * alpha + wave_sum(p);
+      for (int i = 0; i < ND; i++) o[i] *= alpha;
+#pragma unroll 1
+      for (int j = 0; j < min(64, hi - k0); j++) {
+        const float pj = __shfl(p, j);
+        for (int i = 0; i < ND; i++)
+          o[i] = fmaf(pj, values[(size_t)(k0 + j) * kv_dim + lane + 64 * i], o[i]);
+      }
+      m = m_new;
+    }
+    const float g = gate != nullptr ? 1.0f / (1.0f + expf(-gate[th])) : 1.0f;
+    float* w = splits > 1 ? ws + (th * splits + split) * (HD + 4) : nullptr;
+    for (int i = 0; i < ND; i++) {
+      if (w != nullptr) w[4 + lane + 64 * i] = o[i];
+      else out[th * HD + lane + 64 * i] = gate != nullptr ? (o[i] / l) * g : o[i] / l;
+    }
+    if (w != nullptr && lane < 2) w[lane] = lane == 0 ? m : l;
+  }
+}
+
 template <int HD, int GW>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 2)))
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 3)))
 attention_prefill_kernel(const float* __restrict__ q, const float* __restrict__ keys,
                          const float* __restrict__ values, const float* __restrict__ gate,
                          float* __restrict__ out, float* __restrict__ ws, int position, int n,
                          int heads, int kv_dim, int group, int window, float scale, int splits,
                          int tiles_per_split) {
-  constexpr int QW = 4 / GW;
-  constexpr int KS = HD + 4;                     // K row stride in LDS (floats)
-  constexpr int VS = kPK + 4;                    // V^T row stride
-  constexpr int kF4 = HD * kPK / 4 / kThreads;   // float4 per thread per tile and matrix
-  constexpr int kLds = kPK * KS + HD * VS;
-  static_assert(kLds >= 4 * kPQ * (HD + 4), "the output transpose reuses the tiles' LDS");
-  __shared__ __align__(16) float lds[kLds];
-  float* Ks = lds;
-  float* Vt = lds + kPK * KS;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int c16 = lane & 15, g4 = lane >> 4;
+  using T = PrefillTile<HD>;
+  constexpr int KT = T::KT, NS = KT / 16, NE = HD / 16;
+  constexpr int QW = 4 / GW;                     // query blocks of a workgroup
+  __shared__ __align__(16) uint8_t lds[T::kK + T::kV];
+  __shared__ int special[2];   // tile t (t % 2) holds an infinity or NaN
+  uint8_t* Kp = lds;
+  uint8_t* Vp = lds + T::kK;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g4 = lane >> 4;
   const int head = blockIdx.x * GW + wave % GW;
   const int split = blockIdx.z;
-  // Odd splits take the query blocks in reverse: workgroups dispatched
-  // together then pair a late block's long key runs with an early block's
-  // short ones (causal work grows with the block).
-  const int yb = split & 1 ? gridDim.y - 1 - blockIdx.y : blockIdx.y;
+  // The last query blocks have the most keys: they start first.
+  const int yb = gridDim.y - 1 - blockIdx.y;
   const int t0 = (yb * QW + wave / GW) * kPQ;   // the wave's first token
-  // The workgroup's keys: from its first query's window start through its
-  // last query.
   const int wq_first = yb * QW * kPQ;
   const int wq_last = min(n, wq_first + QW * kPQ) - 1;
-  const int kend = position + wq_last + 1;
-  const int kstart = window > 0 ? max(0, position + wq_first - window + 1) : 0;
-  const int ntiles = (kend - kstart + kPK - 1) / kPK;
+  const KeyRange kr = key_range(position, wq_first, wq_last, window);
+  const int ntiles = (kr.end - kr.start + KT - 1) / KT;
   const int tile_lo = split * tiles_per_split;
   const int tile_hi = min(ntiles, tile_lo + tiles_per_split);
+  if (tile_lo >= tile_hi) return;   // the whole workgroup
   const size_t kvo = (size_t)(blockIdx.x * GW / group) * HD;
+  const float sl = scale * 1.44269504088896341f;   // scores in units of log2
 
-  // B operand of S^T: the lane's query, dims g4 * HD / 4 + s.
-  const int tq = t0 + c16;
-  const int qpos = position + tq;
-  float qr[HD / 4];
-  {
-    const float* qp = q + ((size_t)min(tq, n - 1) * heads + head) * HD + g4 * (HD / 4);
-#pragma unroll
-    for (int s4 = 0; s4 < HD / 16; s4++) {
-      const float4 v = *(const float4*)(qp + 4 * s4);
-      qr[4 * s4] = v.x;
-      qr[4 * s4 + 1] = v.y;
-      qr[4 * s4 + 2] = v.z;
-      qr[4 * s4 + 3] = v.w;
-    }
-  }
-  float m_run = -INFINITY, l_run = 0.0f;
-  v4f o[HD / 16];
-#pragma unroll
-  for (int e = 0; e < HD / 16; e++) o[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-
-  // Tile t's keys and values, thread-strided float4s; rows past the keys
-  // read zeros (the resource ends with the last key row).
-  float4 kp[kF4], vp[kF4];
+  // Staging: the first half of the workgroup carries V (thread: 4 dims of the
+  // 8 keys of a key group), the second K (thread: 4 times 8 dims of a key).
+  const bool v_half = wave < 2;
+  const int su = tid & 127;
+  const int vd = su % (HD / 4), vg = su / (HD / 4);   // V: dims 4 vd.., key group vg
+  float4 raw[8];
+  // A resource per row of a thread's eight loads, so that one offset serves
+  // them all; rows past the keys read zeros.
+  const int v_off = (32 * (vg >> 2) + 4 * (vg & 3)) * kv_dim * 4 + vd * 16;
+  const int k_off = su / (HD / 8) * kv_dim * 4 + su % (HD / 8) * 32;
   auto load_tile = [&](int t) {
-    const int kt = kstart + t * kPK;
-    const uint32_t range = (uint32_t)min(kPK, kend - kt) * (uint32_t)kv_dim * 4u;
-    const i32x4 kr = buffer_rsrc(keys + (size_t)kt * kv_dim + kvo, range);
-    const i32x4 vr = buffer_rsrc(values + (size_t)kt * kv_dim + kvo, range);
+    const int kt = kr.start + t * KT, rows = min(KT, kr.end - kt);
+    const size_t at = (size_t)kt * kv_dim + kvo;
+    auto row = [&](const float* base, int r) {
+      return buffer_rsrc(base + at + (size_t)r * kv_dim,
+                         (uint32_t)max(0, rows - r) * (uint32_t)kv_dim * 4u);
+    };
+    if (v_half) {
 #pragma unroll
-    for (int j = 0; j < kF4; j++) {
-      // K: consecutive threads along a row. V: consecutive threads down a
-      // column, so that its transposed LDS writes fall in distinct banks.
-      const int f = j * kThreads + tid;
-      kp[j] = buffer_load_f4(kr, (f / (HD / 4)) * kv_dim * 4 + (f % (HD / 4)) * 16);
-      vp[j] = buffer_load_f4(vr, (f % kPK) * kv_dim * 4 + (f / kPK) * 16);
+      for (int j = 0; j < 8; j++)
+        raw[j] = buffer_load_f4(row(values, 16 * (j >> 2) + (j & 3)), v_off);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const i32x4 r = row(keys, j * (128 / (HD / 8)));
+        raw[2 * j] = buffer_load_f4(r, k_off);
+        raw[2 * j + 1] = buffer_load_f4(r, k_off + 16);
+      }
     }
   };
-  if (tile_lo < tile_hi) load_tile(tile_lo);
-  for (int t = tile_lo; t < tile_hi; t++) {
-    __syncthreads();  // every wave is done with the previous tile
+  auto store_tile = [&](int t) {
+    float rest = 0.0f;
+    uint4 p[3];
+    if (v_half) {
 #pragma unroll
-    for (int j = 0; j < kF4; j++) {
-      const int f = j * kThreads + tid;
-      *(float4*)(Ks + (f / (HD / 4)) * KS + (f % (HD / 4)) * 4) = kp[j];
-      const int row = f % kPK, c4 = f / kPK;
-      Vt[(c4 * 4 + 0) * VS + row] = vp[j].x;
-      Vt[(c4 * 4 + 1) * VS + row] = vp[j].y;
-      Vt[(c4 * 4 + 2) * VS + row] = vp[j].z;
-      Vt[(c4 * 4 + 3) * VS + row] = vp[j].w;
-    }
-    __syncthreads();
-    if (t + 1 < tile_hi) load_tile(t + 1);  // in flight during this tile's math
-    const int kt = kstart + t * kPK;
-
-    // S^T for the tile's two 16-key halves, each as two chains (even and
-    // odd steps) so that dependent MFMAs interleave.
-    v4f sa[2][2];
+      for (int d = 0; d < 4; d++) {
+        const float x[8] = {(&raw[0].x)[d], (&raw[1].x)[d], (&raw[2].x)[d], (&raw[3].x)[d],
+                            (&raw[4].x)[d], (&raw[5].x)[d], (&raw[6].x)[d], (&raw[7].x)[d]};
+        rest += split_pieces(x, p);
+        // Rows of four dims, 64 bytes, would meet in the same banks for
+        // threads two apart: the row's place is turned by bits 3, 4 of the dim.
+        const int slot = 4 * vd + (d ^ ((vd >> 1) & 3));
 #pragma unroll
-    for (int c = 0; c < 2; c++) sa[c][0] = sa[c][1] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int s4 = 0; s4 < HD / 16; s4++) {
-#pragma unroll
-      for (int c = 0; c < 2; c++) {
-        const float4 k4 = *(const float4*)(Ks + (c * 16 + c16) * KS + g4 * (HD / 4) + 4 * s4);
-        sa[c][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.x, qr[4 * s4], sa[c][0], 0, 0, 0);
-        sa[c][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.y, qr[4 * s4 + 1], sa[c][1], 0, 0, 0);
-        sa[c][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.z, qr[4 * s4 + 2], sa[c][0], 0, 0, 0);
-        sa[c][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.w, qr[4 * s4 + 3], sa[c][1], 0, 0, 0);
-      }
-    }
-    // Scores of keys kt + 16 c + 4 g4 + v for query tq, masked; online softmax.
-    float p[2][4];
-    float mt = -INFINITY;
-#pragma unroll
-    for (int c = 0; c < 2; c++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int kpos = kt + c * 16 + 4 * g4 + v;
-        const bool ok = kpos < kend && kpos <= qpos && (window <= 0 || kpos > qpos - window);
-        const float x = (sa[c][0][v] + sa[c][1][v]) * scale;
-        p[c][v] = ok ? x : -INFINITY;
-        mt = fmaxf(mt, p[c][v]);
-      }
-    mt = rows4_max(mt);
-    const float m_new = fmaxf(m_run, mt);
-    const float alpha = m_run == -INFINITY ? 0.0f : __expf(m_run - m_new);
-    float ps = 0.0f;
-#pragma unroll
-    for (int c = 0; c < 2; c++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        p[c][v] = p[c][v] == -INFINITY ? 0.0f : __expf(p[c][v] - m_new);
-        ps += p[c][v];
-      }
-    ps = rows4_sum(ps);
-    l_run = l_run * alpha + ps;
-    // The running sums change only where a max grew (alpha < 1); once the
-    // maxima settle most tiles skip the rescale of the accumulators.
-    if (__any(alpha != 1.0f)) {
-#pragma unroll
-      for (int e = 0; e < HD / 16; e++) o[e] *= alpha;
-    }
-    m_run = m_new;
-    // O^T += V^T P^T: step s takes keys (s / 4) * 16 + 4 g4 + s % 4.
-#pragma unroll
-    for (int c = 0; c < 2; c++) {
-      float4 v4[HD / 16];
-#pragma unroll
-      for (int e = 0; e < HD / 16; e++)
-        v4[e] = *(const float4*)(Vt + (e * 16 + c16) * VS + c * 16 + 4 * g4);
-#pragma unroll
-      for (int e = 0; e < HD / 16; e++)
-        o[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4[e].x, p[c][0], o[e], 0, 0, 0);
-#pragma unroll
-      for (int e = 0; e < HD / 16; e++)
-        o[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4[e].y, p[c][1], o[e], 0, 0, 0);
-#pragma unroll
-      for (int e = 0; e < HD / 16; e++)
-        o[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4[e].z, p[c][2], o[e], 0, 0, 0);
-#pragma unroll
-      for (int e = 0; e < HD / 16; e++)
-        o[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4[e].w, p[c][3], o[e], 0, 0, 0);
-    }
-  }
-
-  // The wave's O^T (dims x 16 queries) through LDS to rows, then out.
-  __syncthreads();  // the tiles' LDS is free
-  float* tw = lds + wave * kPQ * (HD + 4);
-#pragma unroll
-  for (int e = 0; e < HD / 16; e++)
-#pragma unroll
-    for (int v = 0; v < 4; v++) tw[c16 * (HD + 4) + e * 16 + 4 * g4 + v] = o[e][v];
-  if (g4 == 0) {
-    tw[c16 * (HD + 4) + HD] = m_run;
-    tw[c16 * (HD + 4) + HD + 1] = l_run;
-  }
-  __syncthreads();
-  constexpr int kC4 = HD / 4;            // float4 per row
-  constexpr int kRows = 64 / kC4;        // rows per pass of the wave
-  const int c4 = lane % kC4;
-  for (int r = lane / kC4; r < kPQ; r += kRows) {
-    const int tok = t0 + r;
-    if (tok >= n) break;
-    const float* row = tw + r * (HD + 4);
-    const float4 val = *(const float4*)(row + 4 * c4);
-    const size_t th = (size_t)tok * heads + head;
-    if (splits > 1) {
-      float* w = ws + (th * splits + split) * (HD + 4);
-      *(float4*)(w + 4 + 4 * c4) = val;
-      if (c4 == 0) {
-        w[0] = row[HD];
-        w[1] = row[HD + 1];
+        for (int i = 0; i < 3; i++)
+          *(uint4*)(Vp + (i * (KT / 8) + vg) * T::VS + slot * 16) = p[i];
       }
     } else {
-      const float l = row[HD + 1];
-      const float g = gate != nullptr ? 1.0f / (1.0f + expf(-gate[th])) : 1.0f;
-      float4 y = make_float4(val.x / l, val.y / l, val.z / l, val.w / l);
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int u = j * 128 + su, key = u / (HD / 8), g = u % (HD / 8);
+        const float x[8] = {raw[2 * j].x,     raw[2 * j].y,     raw[2 * j].z,     raw[2 * j].w,
+                            raw[2 * j + 1].x, raw[2 * j + 1].y, raw[2 * j + 1].z, raw[2 * j + 1].w};
+        rest += split_pieces(x, p);
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+          *(uint4*)(Kp + (i * (HD / 8) + g) * T::KS + key * 16) = p[i];
+      }
+    }
+    if (!(fabsf(rest) < INFINITY)) special[t & 1] = 1;
+  };
+
+  // B operand of S^T: the lane's query, dims 32 s + 8 g4 + 0..7, in pieces.
+  const int tq = t0 + l16;
+  const int qpos = position + tq;
+  float4 qv[HD / 16];
+  {
+    const float* qp = q + ((size_t)min(tq, n - 1) * heads + head) * HD + 8 * g4;
+#pragma unroll
+    for (int s = 0; s < HD / 32; s++) {
+      qv[2 * s] = *(const float4*)(qp + 32 * s);
+      qv[2 * s + 1] = *(const float4*)(qp + 32 * s + 4);
+    }
+  }
+  load_tile(tile_lo);
+  uint4 qf[HD / 32][3];
+  bool plain;   // an infinity or NaN was met: the wave's rows are formed anew
+  {
+    float rest = 0.0f;
+#pragma unroll
+    for (int s = 0; s < HD / 32; s++) {
+      const float4 a = qv[2 * s], b = qv[2 * s + 1];
+      const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      rest += split_pieces(x, qf[s]);
+    }
+    plain = __any(!(fabsf(rest) < INFINITY));
+  }
+  // The keys that the lane's query sees: see_lo .. see_lo + see_n - 1.
+  const uint32_t see_lo = window > 0 ? max(0, qpos - window + 1) : 0;
+  const uint32_t see_n = min(kr.end - 1, qpos) + 1 - see_lo;
+  float m_run = -INFINITY, l_run = 0.0f;
+  v4f o[NE];
+#pragma unroll
+  for (int e = 0; e < NE; e++) o[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  if (tid < 2) special[tid] = 0;
+
+  for (int t = tile_lo; t < tile_hi; t++) {
+    __syncthreads();  // every wave is done with the previous tile
+    store_tile(t);
+    __syncthreads();
+    if (t + 1 < tile_hi) load_tile(t + 1);  // in flight during this tile's math
+    const bool tile_special = special[t & 1] != 0;
+    if (tid == 0) special[(t + 1) & 1] = 0;   // its last readers are past the barriers
+    const int kt = kr.start + t * KT;
+    const int q_hi = position + min(t0 + kPQ, n) - 1;   // the wave's last query's place
+    if (t0 >= n || kt > q_hi) continue;                 // no query of the wave sees a key
+    plain |= tile_special;
+
+    // Scores of keys kt + 16 u + 4 g4 + v.
+    v4f s[NS];
+#pragma unroll
+    for (int u = 0; u < NS; u++) s[u] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int d = 0; d < HD / 32; d++) {
+#pragma unroll
+      for (int u = 0; u < NS; u++) {
+        uint4 kf[3];
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+          kf[i] = *(const uint4*)(Kp + (i * (HD / 8) + 4 * d + g4) * T::KS + (16 * u + l16) * 16);
+        s[u] = mfma_pieces(kf, qf[d], s[u]);
+      }
+    }
+    const bool edge = kt + KT > position + t0 + 1 || kt + KT > kr.end ||
+                      (window > 0 && kt <= q_hi - window);
+    float mt = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < NS; u++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        if (edge) {
+          const uint32_t key = kt + 16 * u + 4 * g4 + v;
+          s[u][v] = key - see_lo < see_n ? s[u][v] : -INFINITY;
+        }
+        mt = fmaxf(mt, s[u][v]);
+      }
+    mt = rows4_max(mt) * sl;
+    const float m_new = fmaxf(m_run, mt);
+    const float m_ref = m_new == -INFINITY ? 0.0f : m_new;   // nothing seen yet: all p are 0
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_ref);
+    float ps = 0.0f;
+#pragma unroll
+    for (int u = 0; u < NS; u++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        s[u][v] = __builtin_amdgcn_exp2f(fmaf(s[u][v], sl, -m_ref));
+        ps += s[u][v];
+      }
+    l_run = l_run * alpha + rows4_sum(ps);
+    m_run = m_new;
+    uint4 pf[KT / 32][3];
+#pragma unroll
+    for (int h = 0; h < KT / 32; h++) {   // 32 keys
+      float x[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++) x[j] = s[2 * h + (j >> 2)][j & 3];
+      split_pieces(x, pf[h]);
+    }
+    // A tile's sums start from zero and join the running ones in one
+    // multiply-add (with the rescale): one rounding a tile of a long run.
+#pragma unroll
+    for (int e = 0; e < NE; e++) {
+      v4f d = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int h = 0; h < KT / 32; h++) {
+        uint4 vf[3];
+        const int slot = e * 16 + (l16 ^ ((2 * e + (l16 >> 3)) & 3));
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+          vf[i] = *(const uint4*)(Vp + (i * (KT / 8) + 4 * h + g4) * T::VS + slot * 16);
+        d = mfma_pieces(vf, pf[h], d);
+      }
+#pragma unroll
+      for (int v = 0; v < 4; v++) o[e][v] = fmaf(o[e][v], alpha, d[v]);
+    }
+  }
+  if (plain) {
+    prefill_plain<HD>(q, keys + kvo, values + kvo, gate, out, ws, position, n, heads, head, kv_dim,
+                      window, sl, t0, kr.start + tile_lo * KT, min(kr.end, kr.start + tile_hi * KT),
+                      splits, split, lane);
+    return;
+  }
+  // The lane's query, dims 16 e + 4 g4 + 0..3: 64 bytes of a row per store
+  // and query.
+  if (tq >= n) return;
+  const size_t th = (size_t)tq * heads + head;
+  if (splits > 1) {
+    float* w = ws + (th * splits + split) * (HD + 4);
+#pragma unroll
+    for (int e = 0; e < NE; e++)
+      *(float4*)(w + 4 + e * 16 + 4 * g4) = make_float4(o[e][0], o[e][1], o[e][2], o[e][3]);
+    if (g4 == 0) {
+      w[0] = m_run;
+      w[1] = l_run;
+    }
+  } else {
+    const float g = gate != nullptr ? 1.0f / (1.0f + expf(-gate[th])) : 1.0f;
+#pragma unroll
+    for (int e = 0; e < NE; e++) {
+      float4 y = make_float4(o[e][0] / l_run, o[e][1] / l_run, o[e][2] / l_run, o[e][3] / l_run);
       if (gate != nullptr) y = make_float4(y.x * g, y.y * g, y.z * g, y.w * g);
-      *(float4*)(out + th * HD + 4 * c4) = y;
+      *(float4*)(out + th * HD + e * 16 + 4 * g4) = y;
     }
   }
 }
 
-// The combine for many (token, head) rows and at most 64 splits (prefill):
-// one wave per row, four rows per workgroup, no barrier. Lane s holds split
-// s's statistics; the value sums run in split order with C splits' loads in
-// flight (the fewest of 2, 4, 8 covering the splits), dims lane + 64 i. Rows past the splits read zeros (the resource
-// ends with the row's last split), and dims past hd are computed but not
-// stored.
+// How the prefill kernel dealt a row's keys: workgroups of `queries` tokens,
+// tiles of kt keys, tps tiles to a split. A row's last splits may be empty
+// (its keys end before them): they were not written and are not read.
+struct RowSplits {
+  int position, n, window, queries, kt, tps;
+};
+
+// The combine of the prefill kernel's partial rows (at most 64 splits, hd 64
+// or 128): one wave per row, four rows per workgroup, no barrier. Lane s
+// holds split s's statistics, reduced by DPP; lane i sums dims ND i .. ND i +
+// ND - 1 in split order, C splits' loads in flight (the fewest of 2, 4, 8
+// covering the splits), the first C requested with the statistics, so that a
+// row of up to C splits waits for memory once. Splits past the row's last
+// read zeros (the resource ends there).
 //
-// With `panel` (hd a multiple of 32, at most 256), each row's values also go
-// into the fp6 activation panel of out ([tokens][heads * hd]) for the matmul
-// that reads it (a prefill chunk's o projection): the row through the wave's
-// LDS, then four lanes per 32-value block (panel4_lane, the panel
-// quantizer's bytes). Records of tokens past the last row are not written.
-template <int C>  // splits per load batch: 2, 4 or 8
+// With `panel`, each row's values also go into the fp6 activation panel of
+// out ([tokens][heads * hd]) for the matmul that reads it (a prefill chunk's
+// o projection): the row through the wave's LDS, then four lanes per 32-value
+// block (panel4_lane, the panel quantizer's bytes). Records of tokens past
+// the last row are not written.
+template <int C, int ND>  // splits per load batch: 2, 4 or 8; hd / 64
 __global__ void __launch_bounds__(kThreads)
 attention_combine_rows_kernel(const float* __restrict__ ws, const float* __restrict__ gate,
-                              float* __restrict__ out, int heads, int hd, int splits, int rows,
-                              uint8_t* __restrict__ panel) {
-  __shared__ __align__(16) float row_lds[kWaves][256];
-  const int lane = threadIdx.x & 63;
-  const int r = blockIdx.x * kWaves + (threadIdx.x >> 6);   // token * heads + head
+                              float* __restrict__ out, int heads, int max_splits, int rows,
+                              uint8_t* __restrict__ panel, RowSplits rsp) {
+  constexpr int hd = 64 * ND, row = hd + 4;
+  __shared__ __align__(16) float row_lds[kWaves][hd];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = blockIdx.x * kWaves + wave;   // token * heads + head
   if (r >= rows) return;
-  const int row = hd + 4;
-  const i32x4 rs = buffer_rsrc(ws + (size_t)r * splits * row, (uint32_t)splits * row * 4u);
-  const float m = lane < splits ? __int_as_float(dnx_raw_buffer_load_i32(rs, lane * row * 4, 0, 0))
-                                : -INFINITY;
-  const float ls = __int_as_float(dnx_raw_buffer_load_i32(rs, (lane * row + 1) * 4, 0, 0));
-  constexpr int kND = 4;   // dims per lane: hd <= 256
-  const int nd = (hd + 63) / 64;
-  float acc[kND] = {0.0f, 0.0f, 0.0f, 0.0f};
-  const float mx = wave_max(m);
-  const float f = m == -INFINITY ? 0.0f : expf(m - mx);
-  const float l = wave_sum(ls * f);
-  for (int s0 = 0; s0 < splits; s0 += C) {
-    float v[C][kND];
-#pragma unroll
-    for (int u = 0; u < C; u++)
-#pragma unroll
-      for (int i = 0; i < kND; i++)
-        v[u][i] = i < nd ? __int_as_float(dnx_raw_buffer_load_i32(
-                               rs, ((s0 + u) * row + 4 + lane + 64 * i) * 4, 0, 0))
-                         : 0.0f;
+  const int token = r / heads;
+  const int first = token / rsp.queries * rsp.queries;
+  const int splits = live_splits(
+      key_range(rsp.position, first, min(rsp.n, first + rsp.queries) - 1, rsp.window), rsp.kt,
+      rsp.tps);
+  const i32x4 rs = buffer_rsrc(ws + (size_t)r * max_splits * row, (uint32_t)splits * row * 4u);
+  const i32x2 ml = dnx_raw_buffer_load_v2i32(rs, lane * row * 4, 0, 0);
+  float v[C][ND];
+  auto load = [&](int s0) {
 #pragma unroll
     for (int u = 0; u < C; u++) {
-      const float fs = __shfl(f, s0 + u);   // 0 past the last split
+      const int off = ((s0 + u) * row + 4 + ND * lane) * 4;
+      if constexpr (ND == 2) {
+        const i32x2 x = dnx_raw_buffer_load_v2i32(rs, off, 0, 0);
+        v[u][0] = __int_as_float(x.x);
+        v[u][1] = __int_as_float(x.y);
+      } else {
+        v[u][0] = __int_as_float(dnx_raw_buffer_load_i32(rs, off, 0, 0));
+      }
+    }
+  };
+  load(0);
+  const float m = lane < splits ? __int_as_float(ml.x) : -INFINITY;
+  const float mx = wave_max_dpp(m);
+  const float f = m == -INFINITY ? 0.0f : exp2f(m - mx);   // m in units of log2
+  const float l = wave_sum_dpp(__int_as_float(ml.y) * f);
+  float acc[ND] = {};
+  for (int s0 = 0; s0 < splits; s0 += C) {
+    if (s0 > 0) load(s0);
 #pragma unroll
-      for (int i = 0; i < kND; i++) acc[i] += v[u][i] * fs;
+    for (int u = 0; u < C; u++) {
+      const float fs = lane_value(f, s0 + u);   // 0 past the last split
+#pragma unroll
+      for (int i = 0; i < ND; i++) acc[i] += v[u][i] * fs;
     }
   }
   const float g = gate != nullptr ? 1.0f / (1.0f + expf(-gate[r])) : 1.0f;
-  float* mine = row_lds[threadIdx.x >> 6];
 #pragma unroll
-  for (int i = 0; i < kND; i++) {
-    const int d = lane + 64 * i;
-    const float o = gate != nullptr ? (acc[i] / l) * g : acc[i] / l;
-    if (i < nd && d < hd) {
-      out[(size_t)r * hd + d] = o;
-      mine[d] = o;
-    }
+  for (int i = 0; i < ND; i++) acc[i] = gate != nullptr ? (acc[i] / l) * g : acc[i] / l;
+  float* mine = row_lds[wave];
+  float* y = out + (size_t)r * hd + ND * lane;
+  if constexpr (ND == 2) {
+    *(float2*)y = make_float2(acc[0], acc[1]);
+    *(float2*)(mine + 2 * lane) = make_float2(acc[0], acc[1]);
+  } else {
+    *y = acc[0];
+    mine[lane] = acc[0];
   }
   if (panel == nullptr) return;
   // LDS operations of one wave execute in order; the fence keeps the
@@ -1101,7 +1291,7 @@ attention_combine_rows_kernel(const float* __restrict__ ws, const float* __restr
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   __builtin_amdgcn_wave_barrier();
   if (lane < hd / 8) {
-    const int token = r / heads, head = r - token * heads;
+    const int head = r - token * heads;
     const int B = heads * hd / kBlock;
     const int b = head * (hd / kBlock) + (lane >> 2);
     const float4 v0 = *(const float4*)(mine + lane * 8);
@@ -1109,6 +1299,71 @@ attention_combine_rows_kernel(const float* __restrict__ ws, const float* __restr
     panel4_lane(v0, v1, lane & 3, token % kTokens,
                 panel + ((size_t)(token / kTokens) * B + b) * kRec);
   }
+}
+
+template <int HD>
+void launch_combine_rows(const float* ws, const float* gate, float* out, int64_t heads, int splits,
+                         int64_t rows, uint8_t* panel, RowSplits rsp, hipStream_t st) {
+  constexpr int ND = HD / 64;
+  auto k = splits <= 2 ? attention_combine_rows_kernel<2, ND>
+         : splits <= 4 ? attention_combine_rows_kernel<4, ND> : attention_combine_rows_kernel<8, ND>;
+  hipLaunchKernelGGL(k, dim3((unsigned)((rows + kWaves - 1) / kWaves)), dim3(kThreads), 0, st, ws,
+                     gate, out, (int)heads, splits, (int)rows, panel, rsp);
+}
+
+// How the prefill attention deals its keys to workgroups: `splits` runs of
+// tps tiles each (1: the whole range, no workspace), and whether the combine
+// can also write the fp6 panel of the output.
+struct PrefillSplit {
+  int splits, tps;
+  bool panel;
+};
+
+PrefillSplit prefill_split(int64_t position, int64_t n, int64_t heads, int64_t hd, int64_t window,
+                           int gw, int kt) {
+  // Tiles of `keys` keys that a block of `queries` tokens walks.
+  auto tiles_of = [&](int64_t b, int64_t queries, int64_t keys) {
+    const int64_t first = b * queries, last = (first + queries < n ? first + queries : n) - 1;
+    const int64_t from = window > 0 && position + first - window + 1 > 0
+                             ? position + first - window + 1 : 0;
+    return (position + last + 1 - from + keys - 1) / keys;
+  };
+  // Calls with 512 or more blocks of 64 (query, head) pairs, or fewer than 4
+  // tiles of 32 keys, keep their keys whole and need no workspace. The panel
+  // is offered where those blocks, brought to 512 by splitting runs of at
+  // least two such tiles, have at most 64 splits.
+  const int64_t q64 = 64 / gw, blocks64 = (n + q64 - 1) / q64;
+  int64_t longest = 1;
+  for (int64_t b = 0; b < blocks64; b++) longest = std::max(longest, tiles_of(b, q64, 32));
+  const int64_t units = heads / gw * blocks64;
+  int64_t splits32 = 1;
+  if (units < 512 && longest >= 4) {
+    splits32 = std::min((512 + units - 1) / units, longest / 2);
+    const int64_t run = (longest + splits32 - 1) / splits32;
+    splits32 = (longest + run - 1) / run;
+    if (n * heads * splits32 * (hd + 4) * 4 > (1ll << 30) || splits32 > 4096) splits32 = 1;
+  }
+  const int64_t qb = kPQ * (4 / gw), by = (n + qb - 1) / qb;
+  int64_t tmax = 1, total = 0;
+  for (int64_t b = 0; b < by; b++) {
+    const int64_t t = tiles_of(b, qb, kt);
+    tmax = std::max(tmax, t);
+    total += t;
+  }
+  total *= heads / gw;
+  if (splits32 == 1) return {1, (int)tmax, false};
+  // Runs of equal length that make about kTargetWorkgroups of them (two to a
+  // CU; 256, 384, 640 .. 1536 were slower or equal at 17 shapes), at most 64 to a row (the row combine's lanes) and 1 GiB of partials.
+  constexpr int64_t kTargetWorkgroups = 512;
+  int64_t tps = (total + kTargetWorkgroups - 1) / kTargetWorkgroups;
+  tps = std::max(tps, (tmax + 63) / 64);
+  if (tps >= tmax) tps = std::max<int64_t>(1, (tmax + 1) / 2);
+  int64_t splits = (tmax + tps - 1) / tps;
+  while (splits > 2 && n * heads * splits * (hd + 4) * 4 > (1ll << 30)) {
+    tps *= 2;
+    splits = (tmax + tps - 1) / tps;
+  }
+  return {(int)splits, (int)tps, splits32 <= 64 && splits > 1};
 }
 
 template <int HD>
@@ -1452,62 +1707,39 @@ static int attention_impl(const float* q, const float* keys, const float* values
   const int64_t last = position + n - 1;
   const int64_t keys_of_last = window > 0 && last >= window ? window : last + 1;
   const float scale = (float)(1.0 / sqrt((double)hd));
-  // 8+ tokens at hd 64 or 128: the matrix-core kernel, its keys split over
-  // workgroups while fewer than kTargetWaves waves would run.
+  // 8+ tokens at hd 64 or 128: the matrix-core kernel.
   if ((hd == 64 || hd == 128) && n >= 8 && kv_heads * hd <= (1 << 20) &&
       ((uintptr_t)out & 15) == 0) {
-    constexpr int64_t kTargetWaves = 2048;
     const int64_t group = heads / kv_heads;
     const int gw = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
-    const int64_t qb = kPQ * (4 / gw);   // queries per workgroup
-    const int64_t by = (n + qb - 1) / qb;
-    int64_t tmax = 1;  // tiles of the longest workgroup range
-    for (int64_t b = 0; b < by; b++) {
-      const int64_t first = b * qb, lastq = (first + qb < n ? first + qb : n) - 1;
-      const int64_t ks = window > 0 && position + first - window + 1 > 0
-                             ? position + first - window + 1 : 0;
-      const int64_t t = (position + lastq + 1 - ks + kPK - 1) / kPK;
-      if (t > tmax) tmax = t;
-    }
-    const int64_t waves = heads / gw * by * 4;
-    int64_t splits = 1;
-    if (waves < kTargetWaves && tmax >= 4) {
-      splits = (kTargetWaves + waves - 1) / waves;
-      if (splits > tmax / 2) splits = tmax / 2;
-    }
-    int64_t tps = (tmax + splits - 1) / splits;
-    splits = (tmax + tps - 1) / tps;
-    size_t pws = splits > 1 ? (size_t)n * heads * splits * (hd + 4) * 4 : 0;
-    if (pws > ((size_t)1 << 30) || splits > 4096) {
-      splits = 1;
-      tps = tmax;
-      pws = 0;
-    }
-    if (panel != nullptr && !(splits > 1 && splits <= 64)) return DNX_EINVAL;
+    const int kt = hd == 128 ? PrefillTile<128>::KT : PrefillTile<64>::KT;
+    const PrefillSplit sp = prefill_split(position, n, heads, hd, window, gw, kt);
+    if (panel != nullptr && !sp.panel) return DNX_EINVAL;
     float* ws = nullptr;
-    if (splits > 1 && (ws = attention_workspace(pws)) == nullptr) return DNX_ENOMEM;
-    const dim3 grid((unsigned)(heads / gw), (unsigned)by, (unsigned)splits);
+    if (sp.splits > 1 && (ws = attention_workspace((size_t)n * heads * sp.splits * (hd + 4) * 4)) ==
+                             nullptr) {
+      return DNX_ENOMEM;
+    }
+    const int64_t qb = kPQ * (4 / gw);
+    const dim3 grid((unsigned)(heads / gw), (unsigned)((n + qb - 1) / qb), (unsigned)sp.splits);
     const hipStream_t st = (hipStream_t)stream;
     if (hd == 128) {
       launch_prefill<128>(gw, grid, st, q, keys, values, gate, out, ws, (int)position, (int)n,
                           (int)heads, (int)(kv_heads * hd), (int)group, (int)window, scale,
-                          (int)splits, (int)tps);
+                          sp.splits, sp.tps);
     } else {
       launch_prefill<64>(gw, grid, st, q, keys, values, gate, out, ws, (int)position, (int)n,
                          (int)heads, (int)(kv_heads * hd), (int)group, (int)window, scale,
-                         (int)splits, (int)tps);
+                         sp.splits, sp.tps);
     }
     if (hipGetLastError() != hipSuccess) return DNX_ELAUNCH;
-    if (splits > 1 && splits <= 64) {
-      const int64_t rows = n * heads;
-      auto k = splits <= 2 ? attention_combine_rows_kernel<2>
-             : splits <= 4 ? attention_combine_rows_kernel<4> : attention_combine_rows_kernel<8>;
-      hipLaunchKernelGGL(k, dim3((unsigned)((rows + kWaves - 1) / kWaves)), dim3(kThreads), 0, st,
-                         ws, gate, out, (int)heads, (int)hd, (int)splits, (int)rows, panel);
-    } else if (splits > 1) {
-      hipLaunchKernelGGL(attention_combine_kernel<false>, dim3((unsigned)heads, (unsigned)n),
-                         dim3(kThreads), (size_t)splits * 4, st, ws, gate, out, (int)heads,
-                         (int)hd, (int)splits, (float*)nullptr, RopeArgs{});
+    if (sp.splits > 1) {
+      const RowSplits rsp{(int)position, (int)n, (int)window, (int)qb, kt, sp.tps};
+      if (hd == 128) {
+        launch_combine_rows<128>(ws, gate, out, heads, sp.splits, n * heads, panel, rsp, st);
+      } else {
+        launch_combine_rows<64>(ws, gate, out, heads, sp.splits, n * heads, panel, rsp, st);
+      }
     }
     return hipGetLastError() == hipSuccess ? DNX_OK : DNX_ELAUNCH;
   }

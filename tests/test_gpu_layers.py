@@ -118,6 +118,63 @@ def test_attention(gpu_ready, orc, heads, kv, hd, pos, n, window, gated):
     assert ok, err
 
 
+# The edges of the prefill tiles (16 queries a wave, 32 or 64 keys a tile, 32
+# or 64 keys to a product step), of the window, and of the splits.
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("heads,kv,pos,n,window", [
+    (1, 1, 0, 8, 0), (4, 1, 23, 9, 0), (2, 1, 15, 16, 0), (2, 2, 16, 17, 0), (4, 1, 0, 65, 0),
+    (8, 2, 62, 33, 1), (3, 1, 95, 31, 31), (4, 4, 97, 64, 32), (6, 3, 300, 40, 33),
+    (8, 4, 511, 129, 64), (2, 1, 4095, 10, 0), (5, 5, 127, 128, 65)])
+def test_prefill_attention_edges(gpu_ready, orc, heads, kv, pos, n, window, hd):
+    rng = np.random.default_rng(heads + pos + n + hd)
+    q = rng.standard_normal(n * heads * hd).astype(np.float32)
+    keys = rng.standard_normal((pos + n, kv * hd)).astype(np.float32)
+    values = rng.standard_normal((pos + n, kv * hd)).astype(np.float32)
+    out = torch.full((n * heads * hd,), np.nan, device="cuda")
+    D.attention(dev(q), dev(keys), dev(values), None, out, pos, n, heads, kv, hd, window)
+    want = orc.attention(q, keys, values, None, pos, n, heads, kv, hd, window)
+    ok, err = close(host(out), want)
+    assert ok, err
+
+
+@pytest.mark.parametrize("pos,n,hd", [(100, 40, 128), (700, 64, 64), (0, 20, 128)])
+def test_prefill_attention_special_values(gpu_ready, pos, n, hd):
+    """An infinity among the values reaches the tokens that see it and no
+    other; a key whose score is minus infinity counts for nothing; a NaN in a
+    query stays in its rows; values near the largest float stay finite."""
+    heads, kv, total = 4, 2, pos + n
+    rng = np.random.default_rng(pos + n)
+    q = rng.standard_normal((n, heads, hd)).astype(np.float32)
+    keys = rng.standard_normal((total, kv, hd)).astype(np.float32)
+    values = rng.standard_normal((total, kv, hd)).astype(np.float32)
+    q[:, 2:, 5] = np.abs(q[:, 2:, 5]) + 0.1
+    q[3, 0, 7] = np.nan
+    gone, seen = total - n + 2, total - n // 2
+    keys[gone, 1, 5] = -np.inf          # heads 2, 3: score -inf from every query
+    values[seen, 0, 9] = np.inf         # heads 0, 1: from the token at `seen` on
+    values[gone, 1, :] = -3.4e38        # of a key that counts for nothing
+    out = torch.full((n * heads * hd,), 7.0, device="cuda")
+    D.attention(dev(q), dev(keys), dev(values), None, out, pos, n, heads, kv, hd)
+    got = host(out).reshape(n, heads, hd)
+    k64, v64 = keys.astype(np.float64), values.astype(np.float64)
+    k64[gone, 1, 5] = v64[seen, 0, 9] = 0.0
+    for t in range(n):
+        for h in range(heads):
+            s = k64[:pos + t + 1, h // 2] @ q[t, h].astype(np.float64) / np.sqrt(hd)
+            if h >= 2 and gone <= pos + t:
+                s[gone] = -np.inf
+            p = np.exp(s - s.max())
+            want = p / p.sum() @ v64[:pos + t + 1, h // 2]
+            if t == 3 and h == 0:
+                assert np.isnan(got[t, h]).all()
+                continue
+            if h < 2 and seen <= pos + t:
+                assert np.isposinf(got[t, h, 9])
+                want[9] = got[t, h, 9] = 0.0
+            ok, err = close(got[t, h], want.astype(np.float32))
+            assert ok, (t, h, err)
+
+
 def test_attention_limits(gpu_ready):
     lib = _lib.load()
     assert lib.dnx_attention_max_keys(128) >= 15000
