@@ -485,6 +485,199 @@ int launch_skinny(const GemmParams& p, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? DNX_OK : DNX_ELAUNCH;
 }
 
+// ---------------------------------------------------------- chunk (n > 16)
+
+// A prompt chunk (the decoder's 5..64 tokens) in one launch over the whole K:
+// a workgroup owns 32 weight rows and G * 32 tokens, and its 8 waves share K
+// in units of 4 blocks (wave w: units w, w + 8, ...), so a wave's loads of a
+// row use its whole 128-byte lines. Both operands come straight from memory
+// in MFMA order (lane l: row or token l % 32, bytes 16 (l / 32) .. + 15 of a
+// block; a Q4 lane half takes its nibbles of the block's 16 bytes), a unit
+// ahead of the one being multiplied. Per 32 x 32 tile and block one
+// v_mfma_i32_32x32x32_i8 (exact dots), one outer-product MFMA for the scale
+// products, cvt + fma; the waves' sums are added through LDS in wave order
+// (deterministic, whatever G). Blocks past K are skipped by the whole wave.
+//
+// Such a chunk has too little work to fill the chip with 64 x 64 tiles: split
+// over K for that, their partials' round trip and its launch cost more than
+// the products (3072 x 1024 Q8 at 64 tokens: tile + reduce 5.9 + 3.0 us, this
+// 4.0). What bounds it is latency: the launch, one memory round trip per
+// unit, the fold of a wave's blocks and the LDS reduction; its weights alone
+// take 1 us to read.
+// The scale products: all eight K slots of the outer-product MFMA carry a
+// pair of bf16 pieces, so only x2 w2 (2^-32 of the product) is left out and s
+// is the product to float32 rounding, as the skinny kernel's multiply.
+//   half 0: x0 w0 + x0 w1 + x1 w0 + x1 w1, half 1: x0 w2 + x2 w0 + x1 w2 + x2 w1
+DNX_DEV uint2 a_scale8(float x, int half) {
+  uint32_t p0, p1, p2;
+  split3_bf16(x, p0, p1, p2);
+  return half ? make_uint2(p0 | (p2 << 16), p1 | (p2 << 16))
+              : make_uint2(p0 | (p0 << 16), p1 | (p1 << 16));
+}
+DNX_DEV uint2 b_scale8(float w, int half) {
+  uint32_t p0, p1, p2;
+  split3_bf16(w, p0, p1, p2);
+  return half ? make_uint2(p2 | (p0 << 16), p2 | (p1 << 16))
+              : make_uint2(p0 | (p1 << 16), p0 | (p1 << 16));
+}
+
+constexpr int kChunkThreads = 512, kChunkWaves = 8, kUnit = 4;
+
+template <bool kQ4, int G>
+__global__ void __launch_bounds__(kChunkThreads) chunk_kernel(GemmParams p) {
+  __shared__ float red[kChunkWaves][G][16][64];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, c = lane >> 5;
+  const int K = p.cols, B = K / kBlock, M = p.n, N = p.rows;
+  const int n0 = blockIdx.x * 32, m0 = blockIdx.y * (G * 32);
+  const int units = (B + kUnit - 1) / kUnit;
+  constexpr int kFar = -(1 << 20);   // past every operand: reads zeros
+
+  const i32x4 rxq = buffer_rsrc(p.xq, (uint32_t)((size_t)M * K));
+  const i32x4 rqs = buffer_rsrc(p.qs, (uint32_t)((size_t)N * (kQ4 ? K / 2 : K)));
+  const i32x4 rxs = buffer_rsrc(p.xsc, (uint32_t)((size_t)M * B * 4));
+  const i32x4 rws = buffer_rsrc(p.scales, (uint32_t)((size_t)N * B * (kQ4 ? 2 : 4)));
+  // Offsets at block 0; a row past the matrix or the tokens stays far.
+  const int row = n0 + l32;
+  const int offW = row < N ? row * (kQ4 ? K / 2 : K) + (kQ4 ? 0 : 16 * c) : kFar;
+  const int offS = row < N ? row * B * (kQ4 ? 2 : 4) : kFar;
+  int offX[G], offXs[G];
+#pragma unroll
+  for (int g = 0; g < G; g++) {
+    const int m = m0 + g * 32 + l32;
+    offX[g] = m < M ? m * K + 16 * c : kFar;
+    offXs[g] = m < M ? m * B * 4 : kFar;
+  }
+
+  struct Unit {
+    i32x4 w[kUnit], x[G][kUnit];
+    i32x4 ws, xs[G];   // the unit's scales (Q4: raw 16 bits each)
+  };
+  // A unit's last blocks may lie past K: their bytes are another row's and
+  // are not used.
+  auto load = [&](int u, Unit& t) {
+    const int b0 = u < units ? u * kUnit : 0;
+#pragma unroll
+    for (int k = 0; k < kUnit; k++)
+      t.w[k] = dnx_raw_buffer_load_v4i32(rqs, offW + (b0 + k) * (kQ4 ? 16 : 32), 0, 0);
+    if constexpr (kQ4) {
+#pragma unroll
+      for (int k = 0; k < kUnit; k++)
+        t.ws[k] = dnx_raw_buffer_load_i16(rws, offS + (b0 + k) * 2, 0, 0);
+    } else {
+      t.ws = dnx_raw_buffer_load_v4i32(rws, offS + b0 * 4, 0, 0);
+    }
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+#pragma unroll
+      for (int k = 0; k < kUnit; k++)
+        t.x[g][k] = dnx_raw_buffer_load_v4i32(rxq, offX[g] + (b0 + k) * 32, 0, 0);
+      t.xs[g] = dnx_raw_buffer_load_v4i32(rxs, offXs[g] + b0 * 4, 0, 0);
+    }
+  };
+
+  float acc[G][16];
+#pragma unroll
+  for (int g = 0; g < G; g++)
+#pragma unroll
+    for (int v = 0; v < 16; v++) acc[g][v] = 0.0f;
+  auto multiply = [&](int u, const Unit& t) {
+#pragma unroll
+    for (int k = 0; k < kUnit; k++) {
+      if (u * kUnit + k >= B) break;
+      v4i w;
+      if constexpr (kQ4) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const uint32_t q = ((uint32_t)t.w[k][j] >> (4 * c)) & 0x0f0f0f0fu;
+          w[j] = (int)(((q | 0x80808080u) - 0x08080808u) ^ 0x80808080u);   // q - 8
+        }
+      } else {
+        w = v4i{t.w[k][0], t.w[k][1], t.w[k][2], t.w[k][3]};
+      }
+      const uint2 sb =
+          b_scale8(kQ4 ? half_bits_to_float((uint16_t)t.ws[k]) : __int_as_float(t.ws[k]), c);
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        const uint2 sa = a_scale8(__int_as_float(t.xs[g][k]), c);
+        const v4i x = {t.x[g][k][0], t.x[g][k][1], t.x[g][k][2], t.x[g][k][3]};
+        v16i d = {};
+        d = __builtin_amdgcn_mfma_i32_32x32x32_i8(x, w, d, 0, 0, 0);
+        const v16f z = {};
+        const v16f sc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(
+            __builtin_bit_cast(s4, sa), __builtin_bit_cast(s4, sb), z, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[g][v] = fmaf((float)d[v], sc[v], acc[g][v]);
+      }
+    }
+  };
+
+  Unit a, b;
+  load(wave, a);
+  for (int u = wave; u < units; u += 2 * kChunkWaves) {
+    if (u + kChunkWaves < units) load(u + kChunkWaves, b);
+    multiply(u, a);
+    if (u + kChunkWaves >= units) break;
+    if (u + 2 * kChunkWaves < units) load(u + 2 * kChunkWaves, a);
+    multiply(u + kChunkWaves, b);
+  }
+
+#pragma unroll
+  for (int g = 0; g < G; g++)
+#pragma unroll
+    for (int v = 0; v < 16; v++) red[wave][g][v][lane] = acc[g][v];
+  __syncthreads();
+  // Wave w adds outputs w, w + 8 of a lane's 16 per token group.
+  if (row >= N) return;
+#pragma unroll
+  for (int g = 0; g < G; g++)
+#pragma unroll
+    for (int v = wave; v < 16; v += kChunkWaves) {
+      float s = red[0][g][v][lane];
+#pragma unroll
+      for (int w = 1; w < kChunkWaves; w++) s += red[w][g][v][lane];
+      const int m = m0 + g * 32 + (v >> 2) * 8 + c * 4 + (v & 3);
+      if (m < M) store_wt(p.y + (size_t)m * N + row, s);
+    }
+}
+
+// Token groups per workgroup of the chunk kernel for a shape, 0 where the
+// tile kernel is the faster (graph-timed with the quantizer, us, tile kernel
+// against this):
+// * one round of 256 workgroups, or the second round's tail costs more than
+//   the tile kernel's reduce (3072 x 1024 at 200 tokens: 14.6 against 14.4,
+//   6144 x 1024 at 200 14.9 against 20.0);
+// * K <= 1024 (a wave's blocks all requested at once): Q8 3072 x 1024 at 33 /
+//   64 / 128 tokens 9.2 / 10.8 / 12.2 against 7.2 / 7.3 / 9.0, Q4 9.2 / 10.9 /
+//   12.0 against 7.8 / 7.9 / 9.7, 512 x 512 at 17..256 7.7..8.5 against 5.7..6.3;
+// * K <= 2048 (two units a wave) where the launch fills the chip enough: 2048
+//   x 2048 Q8 at 64 / 128 12.8 / 13.7 against 10.2 / 10.4, Q4 12.5 / 13.6
+//   against 11.4 / 11.9; with 64 workgroups or fewer (512 x 2048 Q8 at 64: 9.0
+//   against 9.9), and below 64 tokens of Q4 (2048 x 2048 at 33: 10.1 against
+//   11.3), the tile kernel's K split wins;
+// * longer K: each unit adds a memory round trip (1024 x 3072 at 64: 11.7
+//   against 12.9).
+// Up to 16 tokens the skinny kernel's sums are closer to 64 bits (7.2e-8
+// against 8.4e-8 at K = 1024) and it keeps them.
+int chunk_groups(bool q4, int64_t rows, int64_t cols, int64_t n) {
+  const int64_t blocks = cols / kBlock, row_groups = (rows + 31) / 32;
+  if (n <= 16 || blocks > 64) return 0;
+  for (int g = 1; g <= 2; g++) {
+    const int64_t wgs = row_groups * ((n + 32 * g - 1) / (32 * g));
+    if (wgs > 256) continue;
+    return blocks <= 32 || (wgs > 64 && (!q4 || n >= 64)) ? g : 0;
+  }
+  return 0;
+}
+
+template <bool kQ4, int G>
+int launch_chunk(const GemmParams& p, hipStream_t stream) {
+  const dim3 grid((unsigned)((p.rows + 31) / 32), (unsigned)((p.n + G * 32 - 1) / (G * 32)));
+  hipLaunchKernelGGL((chunk_kernel<kQ4, G>), grid, dim3(kChunkThreads), 0, stream, p);
+  return hipGetLastError() == hipSuccess ? DNX_OK : DNX_ELAUNCH;
+}
+
 // y = the split partials summed in split order (deterministic).
 __global__ void __launch_bounds__(kThreads) splitk_reduce_kernel(const float* __restrict__ part,
                                                                  float* __restrict__ y,
@@ -572,6 +765,10 @@ int launch_gemm(const void* qs, const void* scales, const int8_t* xq, const floa
   // 64 x 64 tiles (2 x 2 waves), which keep ~3 workgroups per CU resident
   // at prefill sizes.
   if (skinny_fits(kQ4, cols, n)) return launch_skinny<kQ4, 1>(p, stream);
+  switch (chunk_groups(kQ4, rows, cols, n)) {
+    case 1: return launch_chunk<kQ4, 1>(p, stream);
+    case 2: return launch_chunk<kQ4, 2>(p, stream);
+  }
   if (n <= 32) return launch_tile<kQ4, 32, 128, 1, 4>(p, stream);
   return launch_tile<kQ4, 64, 64, 2, 4>(p, stream);
 }

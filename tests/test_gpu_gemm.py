@@ -127,6 +127,27 @@ def test_gemm_within_tolerance(gpu_ready, orc, fmt, rows, cols, n, path):
         assert np.all(np.abs(y - ref) <= 1e-4 + 1e-5 * np.abs(ref))
 
 
+# The chunk kernel's edges: 17 tokens (its fewest), whole and ragged groups of
+# 32 tokens and rows, one and two token groups a workgroup, block counts that
+# leave a unit of 4 or a round of 8 units unfilled, and K = 2048. The bar is
+# the one above: error / sum|terms| < 1e-5 (the block dots are exact, each
+# scale product is within 2^-23, and at most 64 float32 additions follow:
+# 66 * 2^-24 = 4e-6).
+@pytest.mark.parametrize("fmt", ["q8", "q4"])
+@pytest.mark.parametrize("rows,cols,n", [(31, 32, 17), (32, 128, 32), (33, 160, 33), (65, 992, 64),
+                                         (3072, 1024, 64), (4000, 1024, 70), (70, 608, 250),
+                                         (2049, 2048, 96), (4096, 1056, 65), (2100, 1120, 64),
+                                         (96, 1024, 1000)])
+def test_chunk_gemm_edges(gpu_ready, orc, fmt, rows, cols, n):
+    print(f"chunk gemm {fmt} {rows}x{cols} n={n}", flush=True)
+    rng = np.random.default_rng(rows + cols + 7 * n)
+    qs, sc = (synth.q8_weights if fmt == "q8" else synth.q4_weights)(rng, rows, cols)
+    xq, xsc = orc.quantize_q8(synth.activations(rng, n, cols))
+    y = gemm(fmt, qs, sc, xq, xsc, rows, cols, n)
+    exact, mag = exact_products(orc, fmt, qs, sc, xq, xsc)
+    assert np.max(np.abs(y - exact) / mag) < 1e-5
+
+
 def test_gemm_rejects_unsupported(gpu_ready):
     z = torch.zeros(4096, device="cuda")
     with pytest.raises(RuntimeError):
