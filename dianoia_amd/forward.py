@@ -80,12 +80,15 @@ def lfm3_small() -> ForwardConfig:
                          conv_kernel=3, sliding_window=3, eps=1e-5, sandwich=True, gate=True)
 
 
-def _rope_row(theta: float, hd: int, position: int) -> tuple[np.ndarray, np.ndarray]:
-    """cos and sin of the hd / 2 rotation angles of one position."""
+def _rope_rows(theta: float, hd: int, position: int, n: int) -> tuple[np.ndarray, np.ndarray]:
+    """cos and sin of the hd / 2 rotation angles of n positions from
+    ``position`` on, a row each. All rows of a chunk in one array operation:
+    a row at a time (64 tokens, two tables) took 500 us of the host's time
+    beside a six-layer chunk's 680 us on the GPU, this about 100."""
     pair = hd // 2
     inv = theta ** (-np.arange(pair, dtype=np.float64) * 2.0 / hd)
-    ang = position * inv
-    return np.cos(ang).astype(np.float32), np.sin(ang).astype(np.float32)
+    ang = np.arange(position, position + n, dtype=np.float64)[:, None] * inv
+    return np.cos(ang), np.sin(ang)
 
 
 class _Buffer:
@@ -344,15 +347,9 @@ class GpuForward:
         lib, c = self.lib, self.config
         h, hd, eps = c.hidden, c.head_dim, c.eps
         pair = hd // 2
-        rope = self._rope.view
-        for t in range(n):
-            fc, fs = _rope_row(c.full_theta, hd, position + t)
-            sc, ss = _rope_row(c.sliding_theta, hd, position + t)
-            at = t * 4 * pair
-            rope[at:at + pair] = fc
-            rope[at + pair:at + 2 * pair] = fs
-            rope[at + 2 * pair:at + 3 * pair] = sc
-            rope[at + 3 * pair:at + 4 * pair] = ss
+        rope = self._rope.view[:n * 4 * pair].reshape(n, 4, pair)
+        rope[:, 0], rope[:, 1] = _rope_rows(c.full_theta, hd, position, n)
+        rope[:, 2], rope[:, 3] = _rope_rows(c.sliding_theta, hd, position, n)
 
         def matmul(w: _Matrix, x: _Buffer, y: int, y_offset: int = 0) -> None:
             f = lib.lab_gpu_enc_matmul_q4 if w.q4 else lib.lab_gpu_enc_matmul_q8
