@@ -209,6 +209,27 @@ def test_q6k_to_q8_matches_oracle(gpu_ready, orc, rows, cols, raw):
     assert np.array_equal(bits(sc), bits(s2))
 
 
+@pytest.mark.parametrize("rows", [8191, 8192])
+def test_q6k_smallest_and_special_scales(gpu_ready, orc, rows):
+    """Finite d down to the smallest fp16 (values of 2^-24 and 0: every scale
+    and its inverse stay normal floats), with infinite and NaN d in the same
+    wave, on either side of the route's 65536 blocks. Bit-exact."""
+    from q6k_util import pack_q6k
+    rng = np.random.default_rng(rows)
+    q = rng.integers(0, 64, size=(rows, 256), dtype=np.uint8)
+    q[:64] = 32                             # all values 0
+    q[64:128, ::32], q[64:128, 1::32] = 33, 31   # one step beside zeros
+    q[64:128, 2::32] = 32
+    sc = rng.choice(np.array([-128, -1, 0, 1, 127], np.int8), size=(rows, 16))
+    d = rng.choice(np.array([0x0001, 0x8001, 0x03FF, 0x0400, 0x7BFF, 0x0000, 0x8000, 0x7C00, 0xFC00,
+                             0x7E00, 0x3C00], np.uint16), size=rows)
+    blocks = pack_q6k(q, sc, d)
+    qs, s = gpu_q6k_to_q8(blocks, rows, 256)
+    q2, s2 = orc.q6k_to_q8(blocks, rows, 256)
+    assert np.array_equal(qs, q2)
+    assert np.array_equal(bits(s), bits(s2))
+
+
 def test_q6k_adapter_through_the_abi(gpu_ready, orc):
     """GpuLinear.upload_q6k -> lab_gpu_enc_q6k_to_q8, then the LM head with the
     fused greedy argmax on the converted weights, bit-exact with the CPU."""
