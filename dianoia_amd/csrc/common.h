@@ -273,7 +273,9 @@ DNX_DEV uint4 buffer_load16_stream(i32x4 rsrc, int offset) {
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 DNX_DEV uint32_t lds_address(const void* p) { return (uint32_t)(size_t)(lds_ptr_t)p; }
 DNX_DEV void buffer_load16_to_lds(i32x4 rsrc, uint32_t lds_addr, int voffset) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+  // One wait state between the write of M0 and the DMA that reads it, which
+  // the compiler's hazard pass would add if it saw them.
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                :
                : "s"(lds_addr), "v"(voffset), "s"(rsrc)
                : "memory");
@@ -284,13 +286,16 @@ DNX_DEV void buffer_load16_to_lds(i32x4 rsrc, uint32_t lds_addr, int voffset) {
 // write-back. For large outputs written once at a kernel's end (a GEMM's
 // 12.6 MB at 512 x 6144) this took the fp6 GEMM from 22.9 to 19.0 us.
 // Inline asm: the compiler does not count these in its wait counters, which
-// only makes its later waits for its own loads stricter.
+// only makes its later waits for its own loads stricter. It does not see the
+// 16-byte store's hazard either: the store still reads its data registers
+// while the next instruction issues, and a VALU write of one of them within
+// two wait states changes what is stored. Hence the s_nop.
 DNX_DEV void store_wt(float* p, float v) {
   asm volatile("global_store_dword %0, %1, off sc0 sc1" : : "v"(p), "v"(v) : "memory");
 }
 DNX_DEV void store_wt4(float* p, float4 v) {
   const f32x4 w = {v.x, v.y, v.z, v.w};
-  asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" : : "v"(p), "v"(w) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" : : "v"(p), "v"(w) : "memory");
 }
 
 DNX_DEV float4 buffer_load_f4(i32x4 rsrc, int offset) {
