@@ -261,6 +261,48 @@ def test_prepacked_gemm_equals_engine_layout(gpu_ready, orc, rows, cols, n):
     assert ok, (worst_rel, worst_abs)
 
 
+@pytest.mark.parametrize("kernel", ["f6", "f6p", "f6s", "i8p", "i8p_wide", "i8p_split"])
+@pytest.mark.parametrize("tail,offset", [(0, 1), (1, 0), (2, 2), (3, 3)])
+def test_outputs_at_any_row_count_and_offset(gpu_ready, orc, kernel, tail, offset):
+    """Outputs stored 16 bytes at a time also where a token's row starts at
+    any float (rows not a multiple of four, y at any float offset): the
+    values, the last rows of each token, and the floats around y untouched."""
+    rows, cols, n = {"f6": (300, 1024, 140), "f6p": (300, 1024, 140), "f6s": (96, 512, 37),
+                     "i8p": (4000, 256, 600), "i8p_wide": (4316, 64, 1000),
+                     "i8p_split": (200, 1024, 130)}[kernel]
+    rows += tail
+    q8 = kernel.startswith("i8p")
+    rng = np.random.default_rng(rows + offset)
+    qs, sc = (synth.q8_weights if q8 else synth.q4_weights)(rng, rows, cols)
+    xs = synth.activations(rng, n, cols)
+    around = torch.full((offset + n * rows + 8,), 7.0, device="cuda")
+    y = around[offset:offset + n * rows]
+    if q8:
+        panel = torch.empty(D.i8_panel_bytes(n, cols), dtype=torch.uint8, device="cuda")
+        packed = torch.empty(D.q8_i8pack_bytes(rows, cols), dtype=torch.uint8, device="cuda")
+        D.quantize_q8_i8panel(dev(xs), panel, n, cols)
+        D.pack_q8_i8(dev(qs), dev(sc), packed, rows, cols)
+        D.gemm_q8_i8p(packed, panel, y, rows, cols, n)
+    else:
+        panel = torch.empty(D.f6_panel_bytes(n, cols), dtype=torch.uint8, device="cuda")
+        packed = torch.empty(D.q4_f6pack_bytes(rows, cols), dtype=torch.uint8, device="cuda")
+        D.quantize_q8_f6panel(dev(xs), panel, n, cols)
+        D.pack_q4_f6(dev(qs), dev(sc), packed, rows, cols)
+        if kernel == "f6":
+            D.gemm_q4_f6(dev(qs), dev(sc), panel, y, rows, cols, n)
+        else:
+            (D.gemm_q4_f6s if kernel == "f6s" else D.gemm_q4_f6p)(packed, panel, y, rows, cols, n)
+    got = host(around)
+    assert (got[:offset] == 7.0).all() and (got[offset + n * rows:] == 7.0).all()
+    got = got[offset:offset + n * rows].reshape(n, rows)
+    ref = (orc.gemm_q8 if q8 else orc.gemm_q4)(qs, sc, xs, n, threads=8, mode=1)
+    if q8:   # outputs of about 30: the reference GPU test's bar, as in test_gpu_gemm.py
+        assert np.all(np.abs(got - ref) <= 1e-4 + 1e-5 * np.abs(ref))
+    else:
+        ok, worst_rel, worst_abs = within_tolerance(got, ref)
+        assert ok, (worst_rel, worst_abs)
+
+
 # ------------------------------------------- the prefill chunk GEMM (5..512 tokens)
 
 def gemm_f6s(qs, sc, xq, xsc, rows, cols, n):
