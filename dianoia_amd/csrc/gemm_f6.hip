@@ -748,8 +748,7 @@ struct F6PParams {
 };
 
 // Stages of kPKB blocks (Q8: kPKB / 2); a stage's weights (SN row groups x
-// its blocks: 24 KB of Q4, 30 KB of Q8, so that two or three workgroups fit
-// a CU's LDS; contiguous per row group in the prepack) move
+// its blocks: 8 KB of Q4 and 10 KB of Q8 a group, contiguous in the prepack) move
 // into one of two LDS buffers by DMA in 1 KB pieces, spread over the waves,
 // issued at the start of the stage before: they arrive while that stage
 // computes. The activation records stay in a register ring one stage
@@ -1213,10 +1212,48 @@ int launch_f6(const uint8_t* qs, const uint16_t* scales, const uint8_t* panel, f
   return DNX_OK;
 }
 
-template <int SN, bool kQ8 = false>
+// The tile of the fp6 prepacked GEMM: SN row groups (32 to 128 rows) per
+// workgroup of 128 tokens, the one whose launch takes the least time by its
+// rounds of 256 workgroups. K is split as for 96-row tiles whatever SN is
+// (dnx_gemm_q4_f6 adds the same partials), and an output's sums do not depend
+// on SN. A block costs a workgroup about 48 ns per row group and as much
+// again for its activations (Q8: 80; measured from 65 to 1024 tokens and 16
+// to 192 blocks); the Q8 kernel of one row group holds 126 registers, so two
+// workgroups share a CU (a round of 512 in 240 ns a block: what two row
+// groups alone cost, so Q8 never takes 64 rows). Over 60 random
+// shapes the chosen tile was at most 1% (Q8 16%) behind the best of the four
+// and never behind 96 rows, which every shape took before: 2048 x 6144 Q4 at
+// 1000 tokens 37.5 -> 31.4 us (64 rows), 6146 x 2048 at 512 33.6 -> 22.9 (128
+// rows: one round, not two), 4096 x 4096 at 1024 53.6 -> 38.0, 768 x 512 at
+// 1024 7.4 -> 4.6 (32 rows); Q8 4096 x 4096 at 1024 84.7 -> 57.5.
+int f6p_row_groups(int64_t rows, int64_t cols, int64_t n, bool q8) {
+  const int64_t tm = (n + kTileM * kTokens - 1) / (kTileM * kTokens);
+  const int64_t gn = (rows + 31) / 32;
+  const int B = (int)(cols / kBlock);
+  const int per = f6_split_blocks((int)(tm * ((gn + 2) / 3)), B);
+  const int64_t splits = (B + per - 1) / per;
+  const double blocks = per < B ? per : B;
+  int best = 3;
+  double best_ns = 0.0;
+  for (int sn = 1; sn <= 4; sn++) {
+    if (q8 && sn == 2) continue;
+    const int64_t wgs = tm * ((gn + sn - 1) / sn) * splits;
+    const bool paired = q8 && sn == 1 && wgs > 256;
+    const double block_ns = paired ? 240.0 : (q8 ? 80.0 : 48.0) * (sn + 1);
+    const int64_t round = paired ? 512 : 256;
+    const double ns = (double)((wgs + round - 1) / round) * (1000.0 + blocks * block_ns);
+    if (sn == 1 || ns < best_ns) {
+      best = sn;
+      best_ns = ns;
+    }
+  }
+  return best;
+}
+
+template <int SN, bool kQ8>
 int launch_f6p(const uint8_t* packed, const uint8_t* panel, float* y, int64_t rows,
-               int64_t cols, int64_t n, hipStream_t stream, float* fixed_part = nullptr,
-               size_t fixed_floats = 0) {
+               int64_t cols, int64_t n, hipStream_t stream, float* fixed_part,
+               size_t fixed_floats) {
   constexpr int BN = SN * 32;
   F6PParams p{};
   p.packed = packed;
@@ -1228,9 +1265,10 @@ int launch_f6p(const uint8_t* packed, const uint8_t* panel, float* y, int64_t ro
   p.tiles_m = (int)((n + kTileM * kTokens - 1) / (kTileM * kTokens));
   p.tiles = p.tiles_m * (int)((rows + BN - 1) / BN);
   const int B = (int)(cols / kBlock);
-  // The same split of K as launch_f6 (whole kKB-block parts, kKB a multiple
-  // of kPKB), so that both kernels add the same partials in the same order.
-  p.split_blocks = f6_split_blocks(p.tiles, B);
+  // The same split of K as launch_f6 (that of its 96-row tiles, in whole
+  // kKB-block parts, kKB a multiple of kPKB), so that both kernels add the
+  // same partials in the same order.
+  p.split_blocks = f6_split_blocks(p.tiles_m * (int)((rows + 95) / 96), B);
   int splits = (B + p.split_blocks - 1) / p.split_blocks;
   const int64_t count = n * rows;
   p.part = nullptr;
@@ -1254,6 +1292,24 @@ int launch_f6p(const uint8_t* packed, const uint8_t* panel, float* y, int64_t ro
     if (hipGetLastError() != hipSuccess) return DNX_ELAUNCH;
   }
   return DNX_OK;
+}
+
+template <bool kQ8>
+int run_f6p(const void* packed, const void* panel, float* y, int64_t rows, int64_t cols,
+            int64_t n, dnx_stream_t stream, float* fixed_part = nullptr,
+            size_t fixed_floats = 0) {
+  const uint8_t* pk = (const uint8_t*)packed;
+  const uint8_t* pn = (const uint8_t*)panel;
+  const hipStream_t st = (hipStream_t)stream;
+  const int sn = f6p_row_groups(rows, cols, n, kQ8);
+  if constexpr (!kQ8) {
+    if (sn == 2) return launch_f6p<2, kQ8>(pk, pn, y, rows, cols, n, st, fixed_part, fixed_floats);
+  }
+  switch (sn) {
+    case 1: return launch_f6p<1, kQ8>(pk, pn, y, rows, cols, n, st, fixed_part, fixed_floats);
+    case 3: return launch_f6p<3, kQ8>(pk, pn, y, rows, cols, n, st, fixed_part, fixed_floats);
+    default: return launch_f6p<4, kQ8>(pk, pn, y, rows, cols, n, st, fixed_part, fixed_floats);
+  }
 }
 
 // ----------------------------------- Q8 weights, prepacked, on int8 MFMA
@@ -1711,8 +1767,7 @@ int dnx_gemm_q4_f6p(const void* packed, const void* panel, float* y, int64_t row
       ((uintptr_t)y & 3)) {
     return DNX_EINVAL;
   }
-  return launch_f6p<3>((const uint8_t*)packed, (const uint8_t*)panel, y, rows, cols, n,
-                       (hipStream_t)stream);
+  return run_f6p<false>(packed, panel, y, rows, cols, n, stream);
 }
 
 int dnx_gemm_q4_f6s(const void* packed, const void* panel, float* y, int64_t rows, int64_t cols,
@@ -1825,8 +1880,7 @@ int dnx_gemm_q8_f6p(const void* packed, const void* panel, float* y, int64_t row
       ((uintptr_t)packed & 15) || ((uintptr_t)y & 3)) {
     return DNX_EINVAL;
   }
-  return launch_f6p<3, true>((const uint8_t*)packed, (const uint8_t*)panel, y, rows, cols, n,
-                             (hipStream_t)stream);
+  return run_f6p<true>(packed, panel, y, rows, cols, n, stream);
 }
 
 int64_t dnx_i8_panel_bytes(int64_t n, int64_t cols) {
@@ -1907,8 +1961,7 @@ int dnx_gemm_q4_f6p_noalloc(const void* packed, const void* panel, float* y, int
   }
   float* part = scratch_on_device();
   if (part == nullptr) return DNX_ESCRATCH;
-  return launch_f6p<3>((const uint8_t*)packed, (const uint8_t*)panel, y, rows, cols, n,
-                       (hipStream_t)stream, part, kScratchFloats);
+  return run_f6p<false>(packed, panel, y, rows, cols, n, stream, part, kScratchFloats);
 }
 
 }  // extern "C"

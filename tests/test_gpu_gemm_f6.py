@@ -261,6 +261,47 @@ def test_prepacked_gemm_equals_engine_layout(gpu_ready, orc, rows, cols, n):
     assert ok, (worst_rel, worst_abs)
 
 
+@pytest.mark.parametrize("q8", [False, True])
+@pytest.mark.parametrize("rows,cols,n", [
+    (161, 512, 385),     # 32 rows a workgroup
+    (2081, 64, 400),     # 64 (Q8: 32, two workgroups a CU)
+    (4227, 96, 513),     # 96
+    (6146, 96, 512),     # 128
+])
+def test_prepacked_gemm_tile_edges(gpu_ready, q8, rows, cols, n):
+    """Every workgroup shape: an output's bits do not depend on the rows and
+    tokens around it (K is not split here), so each slice of the product,
+    cut where the tiles of the whole one end and inside them, equals the
+    product of that slice alone, and nothing past the output is written."""
+    rng = np.random.default_rng(rows + n)
+    if q8:
+        qs, sc = synth.q8_weights(rng, rows, cols)
+        pack, size, run = D.pack_q8_f6, D.q8_f6pack_bytes, D.gemm_q8_f6p
+    else:
+        qs, sc = synth.q4_weights(rng, rows, cols)
+        pack, size, run = D.pack_q4_f6, D.q4_f6pack_bytes, D.gemm_q4_f6p
+    xs = synth.activations(rng, n, cols)
+
+    def product(r0, r1, t0, t1):
+        m, k = r1 - r0, t1 - t0
+        packed = torch.empty(size(m, cols), dtype=torch.uint8, device="cuda")
+        pack(dev(qs[r0:r1]), dev(sc[r0:r1]), packed, m, cols)
+        panel = torch.empty(D.f6_panel_bytes(k, cols), dtype=torch.uint8, device="cuda")
+        D.quantize_q8_f6panel(dev(xs[t0:t1]), panel, k, cols)
+        y = torch.full((k * m + 64,), float("nan"), device="cuda")
+        run(packed, panel, y[:k * m], m, cols, k)
+        out = host(y)
+        assert np.isnan(out[k * m:]).all()
+        return out[:k * m].reshape(k, m)
+
+    whole = product(0, rows, 0, n)
+    assert np.isfinite(whole).all()
+    for r0, r1 in [(0, 33), (31, 97), (95, 161), (rows - 130, rows), (rows - 1, rows)]:
+        for t0, t1 in [(0, 7), (120, 140), (n - 1, n)]:
+            part = product(r0, r1, t0, t1)
+            assert np.array_equal(bits(part), bits(whole[t0:t1, r0:r1])), (r0, r1, t0, t1)
+
+
 @pytest.mark.parametrize("kernel", ["f6", "f6p", "f6s", "i8p", "i8p_wide", "i8p_split"])
 @pytest.mark.parametrize("tail,offset", [(0, 1), (1, 0), (2, 2), (3, 3)])
 def test_outputs_at_any_row_count_and_offset(gpu_ready, orc, kernel, tail, offset):
