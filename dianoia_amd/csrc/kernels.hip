@@ -474,27 +474,40 @@ swiglu_kernel(float* __restrict__ g, const float* __restrict__ u, int64_t count)
 }
 
 // Abramowitz-Stegun 7.1.26 erf in double (lib/src/vision_encoder.dart:
-// 496-509) and the projector's GELU (:260-263), stored to float.
-DNX_DEV double as_erf(double value) {
-  const double x = fabs(value);
-  const double t = 1 / (1 + 0.3275911 * x);
+// 496-509) and the projector's GELU (:260-263), stored to float. The two
+// IEEE divisions, which took a third of the double operations, without
+// their scaling and special cases, none of which the operands need:
+//  - |v| / sqrt 2 as a product with the rounded reciprocal and one residual
+//    step, which rounds as the division does for every float (checked over
+//    all mantissas; the step does not depend on the exponent);
+//  - 1 / d for d in [1, 3.4] by Newton steps from the hardware's reciprocal.
+// |v| above 10 counts as 10: there poly * exp(-x^2) is below 1e-22 and the
+// result 1 either way, and infinities and NaN need no case of their own (v
+// itself enters the last product).
+DNX_DEV float gelu1(float f) {
+  const double v = f;
+  constexpr double kSqrt2 = 1.4142135623730951, kInvSqrt2 = 1 / kSqrt2;
+  const double a = fmin(fabs(v), 10.0);
+  double x = a * kInvSqrt2;
+  x = fma(fma(-x, kSqrt2, a), kInvSqrt2, x);
+  const double d = 1 + 0.3275911 * x;
+  double t = __builtin_amdgcn_rcp(d);
+#pragma unroll
+  for (int k = 0; k < 3; k++) t = fma(fma(-d, t, 1.0), t, t);
   const double poly =
       (((((1.061405429 * t - 1.453152027) * t) + 1.421413741) * t - 0.284496736) * t +
        0.254829592) *
       t;
-  const double result = 1 - poly * exp(-x * x);
-  return value < 0 ? -result : result;
-}
-
-DNX_DEV float gelu1(float f) {
-  const double v = f;
-  return (float)(0.5 * v * (1 + as_erf(v / 1.4142135623730951)));
+  const double erf = 1 - poly * exp(-x * x);
+  return (float)(0.5 * v * (1 + (v < 0 ? -erf : erf)));
 }
 
 // Four values per thread and pass: one 16-byte load and store, and four
-// independent double chains (two IEEE divisions and an exp each) for the
+// independent double chains (a reciprocal and an exp each) for the
 // scheduler to interleave; one value per thread left each wave waiting on
-// one chain (15 us for the vision pair's 4.4 M values). x16 is x from its
+// one chain (15 us for the vision pair's 4.4 M values). Four values took
+// 13.8 us, and 11.6 since the divisions went (35 MB at 3 TB/s): still bound
+// by the double operations, of which exp is half. x16 is x from its
 // first 16-byte aligned value (head values before it, tail values after the
 // last whole quad: done one per thread by workgroup 0).
 __global__ void __launch_bounds__(kThreads) gelu_kernel(float* __restrict__ x, int64_t count,

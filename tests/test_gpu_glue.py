@@ -38,3 +38,21 @@ def test_gelu_bit_exact_at_any_offset(gpu_ready, orc, count, offset):
     assert np.array_equal(np.isnan(got), nan)
     assert np.array_equal(bits(got[~nan]), bits(want[~nan]))
     assert np.all(out[:offset] == 7.0) and np.all(out[offset + count:] == 7.0)
+
+
+@pytest.mark.parametrize("low,high", [(-150, -126), (-30, 3), (3.2, 3.45), (3, 128)])
+def test_gelu_bit_exact_over_magnitudes(gpu_ready, orc, low, high):
+    """Both signs from the denormals to the largest floats, and closely
+    around 10, where the kernel's error function stops following |v|."""
+    rng = np.random.default_rng(17)
+    with np.errstate(over="ignore"):
+        x = np.exp2(rng.uniform(low, high, 1 << 16)).astype(np.float32)
+    x[::2] *= -1
+    ten = np.float32(10.0)
+    x[:4] = [np.nextafter(ten, np.float32(0)), ten, np.nextafter(ten, np.float32(11)), -ten]
+    d = dev(x)
+    D.gelu(d)
+    got, want = host(d), orc.gelu(x)
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(bits(got[~nan]), bits(want[~nan]))
