@@ -652,7 +652,8 @@ def bench_layers(torch, D, timer, steps):
     decode over a 4096-position cache (32 query heads, 8 KV heads, hd 128;
     HBM-bound on the cached keys and values), RMSNorm over a 4096 x 2048
     prefill block, causal prefill attention of 512 tokens (same heads;
-    fp32 matrix cores) and the short convolution at 1 and 512 tokens.
+    fp32 operands as three bf16 pieces, its rate beside the fp32 matrix
+    cores' peak) and the short convolution at 1 and 512 tokens.
     Inputs generated on the GPU."""
     gen = torch.Generator(device="cuda").manual_seed(6)
     heads, kv, hd, pos = 32, 8, 128, 4095
@@ -983,7 +984,7 @@ PMC_KERNELS = {  # kernel-name fragment -> (workload, algorithmic bytes per laun
     "gemm_f6p_kernel<3, true>": (
         "c4 fc1 Q8 fp6 GEMM (prepacked) M=1024, 4320x1152", 4320 * 36 * 80 + 32 * 36 * 2048
         + 1024 * 4320 * 4),
-    "gemm_float_kernel<false, 4>": (
+    "gemm_float_kernel<false": (
         "c4 fc1 float-input Q8 GEMM M=1024, 4320x1152", 4320 * 1152 + 4320 * 36 * 4
         + 1024 * 1152 * 4 + 1024 * 4320 * 4),
 }
@@ -1153,10 +1154,10 @@ MFMA_KERNELS = {
                               2 * 1024 * 4304 * 1152, I8_PEAK_TOPS),
     "gemm_i8p_kernel<4, 4>": ("c4 fc2 Q8 GEMM M=1024 (int8 MFMA, prepacked, 3 K parts)",
                               2 * 1024 * 4304 * 1152, I8_PEAK_TOPS),
-    "gemm_float_kernel<false, 4>": ("c4 fc1 float inputs M=1024 (bf16)",
-                                    2 * 1024 * 4320 * 1152, 2500.0),
+    "gemm_float_kernel<false": ("c4 fc1 float inputs M=1024 (bf16)",
+                                2 * 1024 * 4320 * 1152, 2500.0),
     "attention_prefill_kernel<128, 4>": ("prefill attention 512 tokens, 32/8 heads, hd 128",
-                                         4 * 128 * 32 * (512 * 513 // 2), 157.3),
+                                         4 * 128 * 32 * (512 * 513 // 2), 2500.0 / 6),
 }
 MFMA_COUNTERS = ("SQ_INSTS_MFMA", "SQ_VALU_MFMA_BUSY_CYCLES", "SQ_INSTS_VALU", "SQ_INSTS_LDS",
                  "SQ_LDS_BANK_CONFLICT", "SQ_WAIT_INST_LDS", "SQ_BUSY_CU_CYCLES", "SQ_WAVES")
