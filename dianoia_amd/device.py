@@ -16,8 +16,8 @@ import torch
 from . import _lib
 
 
-# Sizes depend on a shape alone.
-_size = functools.lru_cache(maxsize=1024)
+# Sizes depend on a shape alone. typed: 64.0 is refused also where 64 is held.
+_size = functools.lru_cache(maxsize=1024, typed=True)
 
 
 # A small kernel runs for less time than its launch takes from Python, so the

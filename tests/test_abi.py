@@ -5,7 +5,10 @@ import ctypes
 import os
 import subprocess
 
+import pytest
+
 from dianoia_amd import _lib
+from dianoia_amd import device as D
 
 # The reference's GPU entry points that Dart binds (lib/src/gpu.dart:36-312):
 # the matmul path, everything GpuLinear and the GPU layer's lifecycle,
@@ -56,3 +59,13 @@ def test_no_oracle_in_product():
     assert "lab_oracle" not in out and "lab_native" not in out
     syms = subprocess.run(["nm", "-D", _lib.LIB_PATH], capture_output=True, text=True).stdout
     assert "orc_" not in syms
+
+
+@pytest.mark.parametrize("size", [D.gemm_panel_bytes, D.f6_panel_bytes, D.q4_f6pack_bytes,
+                                  D.q8_f6pack_bytes, D.i8_panel_bytes, D.q8_i8pack_bytes])
+def test_sizes_refuse_floats_also_after_integers(size):
+    """The C ABI takes integers: a float shape is an error whether or not the
+    same number was asked for as an integer before."""
+    assert size(64, 96) > 0
+    with pytest.raises(ctypes.ArgumentError):
+        size(64.0, 96)
