@@ -816,9 +816,12 @@ attention_combine_kernel(const float* __restrict__ ws, const float* __restrict__
 // multiply-add, so a long run rounds once a tile (64 bits say 3.9e-7 after
 // 4000 keys where sums carried through the MFMAs had 9.5e-7).
 // A wave whose queries see no key of a tile skips it; only tiles at the edge
-// of the causal or window range are masked. A wave that meets an
-// infinity or NaN (in Q, or in a tile that it works on) forms its rows anew
-// in plain float32 from memory at the end (slow, and rare).
+// of the causal or window range are masked.
+//
+// An infinity or NaN has no pieces (nor has a float that rounds to an infinity
+// as bf16), and finite terms may overflow with either sign: what they meet
+// comes out as NaN. A wave that ends with an infinity or NaN in its sums forms
+// them anew from memory (prefill_special).
 //
 // With `splits` > 1 a workgroup takes a run of tiles_per_split tiles and
 // writes per (token, head) the partial (m, l, o) rows that
@@ -888,12 +891,11 @@ DNX_DEV float rows4_sum(float v) {
 
 // Eight floats as three bf16 fragments (piece i of value j in element j),
 // each piece the rest rounded to nearest: the terms that are not formed are
-// then as often too small as too large. Returns a finite number, or an
-// infinity or NaN if a value is one (or rounds to one as bf16).
+// then as often too small as too large. An infinity, a NaN and a float that
+// rounds to an infinity have NaN among their pieces.
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-DNX_DEV float split_pieces(const float* x, uint4* p) {
-  float rest = 0.0f;
+DNX_DEV void split_pieces(const float* x, uint4* p) {
   uint32_t w[3][4];
 #pragma unroll
   for (int j = 0; j < 8; j += 2) {
@@ -904,12 +906,10 @@ DNX_DEV float split_pieces(const float* x, uint4* p) {
       if (i == 2) break;
       v.x -= __uint_as_float(w[i][j / 2] << 16);
       v.y -= __uint_as_float(w[i][j / 2] & 0xffff0000u);
-      if (i == 0) rest += v.x + v.y;
     }
   }
 #pragma unroll
   for (int i = 0; i < 3; i++) p[i] = make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]);
-  return rest;
 }
 
 // acc += A B over the six piece products, the smallest first.
@@ -922,51 +922,128 @@ DNX_DEV v4f mfma_pieces(const uint4* a, const uint4* b, v4f acc) {
   return acc;
 }
 
-// The rows of a wave's queries over keys k_lo .. k_hi - 1 in plain float32,
-// for operands that have no pieces (infinities, NaN): a query at a time, a
-// lane to a key for the scores and to HD / 64 dims for the values. Hidden
-// keys count for nothing, whatever they hold.
+// The sums (m, l, o) of a wave's 16 queries over keys k_lo .. k_hi - 1 where
+// an operand has no pieces: the same products on the float32 matrix cores,
+// straight from memory, in the layout of the kernel below (see_lo and see_n:
+// the keys that the lane's query sees). Hidden keys count for nothing,
+// whatever they hold: an infinity or NaN among the values is zero in the
+// products, and a code for it (1: +inf, 128: -inf, 129: NaN) is summed over
+// the keys that are seen, times 1 where p > 0 and 2^14 where p is zero (zero
+// times an infinity is NaN; 32 codes stay below 2^14). Once every sum l is
+// NaN, so is every output, and the rest of the keys is left out.
+//
+// One wave alone walks its keys, so a step's latency is what it costs: 32
+// keys a step in two chains, the next step's keys and this step's values
+// requested before the scores are formed (1000 tokens after 1000, 16 / 8
+// heads, hd 128, us; the finite call takes 110: one infinity among the values
+// 196, 236 with 16 keys a step and nothing ahead, and 4270 as a query at a time
+// in plain loads; every value infinite 369, 424 and 7060; a NaN among the keys
+// 107 to 138, every operand NaN 108 to 120. The float32 matrix cores alone,
+// with the keys shared in LDS, took 170 to 180 whatever the values).
 template <int HD>
-DNX_DEV void prefill_plain(
-    const float* q, const float* keys, const float* values, const float* gate, float* out,
-    float* ws, int position, int n, int heads, int head, int kv_dim, int window, float sl, int t0,
-    int k_lo, int k_hi, int splits, int split, int lane) {
-  constexpr int ND = HD / 64;
+DNX_DEV void prefill_special(const float* qp, const float* keys, const float* values, int kv_dim,
+                             float sl, int k_lo, int k_hi, uint32_t see_lo, uint32_t see_n,
+                             int lane, float& m, float& l, v4f* o) {
+  constexpr int NE = HD / 16, ND = HD / 16, NU = 2;   // NU times 16 keys a step
+  const int l16 = lane & 15, g4 = lane >> 4;
+  m = -INFINITY;
+  l = 0.0f;
+#pragma unroll
+  for (int e = 0; e < NE; e++) o[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  float4 qr[ND], kr[NU][ND];
+#pragma unroll
+  for (int d = 0; d < ND; d++) qr[d] = *(const float4*)(qp + 16 * d + 4 * g4);
+  auto load_keys = [&](int k0) {   // those past the last: the last
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+      const float* kp = keys + (size_t)min(k0 + 16 * u + l16, k_hi - 1) * kv_dim + 4 * g4;
+#pragma unroll
+      for (int d = 0; d < ND; d++) kr[u][d] = *(const float4*)(kp + 16 * d);
+    }
+  };
+  if (k_lo < k_hi) load_keys(k_lo);
 #pragma unroll 1
-  for (int tok = t0; tok < min(t0 + kPQ, n); tok++) {
-    const int qpos = position + tok;
-    const size_t th = (size_t)tok * heads + head;
-    const float* qp = q + th * HD;
-    const int lo = window > 0 ? max(k_lo, qpos - window + 1) : k_lo, hi = min(k_hi, qpos + 1);
-    float m = -INFINITY, l = 0.0f, o[ND] = {};
-#pragma unroll 1
-    for (int k0 = lo; k0 < hi; k0 += 64) {
-      const bool live = k0 + lane < hi;
-      const float* k = keys + (size_t)(live ? k0 + lane : lo) * kv_dim;
-      float s = 0.0f;
-#pragma unroll 1
-      for (int e = 0; e < HD; e++) s = fmaf(k[e], qp[e], s);
-      s = live ? s : -INFINITY;
-      const float m_new = fmaxf(m, wave_max(s) * sl), ref = m_new == -INFINITY ? 0.0f : m_new;
-      const float p = live ? __builtin_amdgcn_exp2f(fmaf(s, sl, -ref)) : 0.0f;
-      const float alpha = __builtin_amdgcn_exp2f(m - ref);
-      l = l * alpha + wave_sum(p);
-      for (int i = 0; i < ND; i++) o[i] *= alpha;
-#pragma unroll 1
-      for (int j = 0; j < min(64, hi - k0); j++) {
-        const float pj = __shfl(p, j);
-        for (int i = 0; i < ND; i++)
-          o[i] = fmaf(pj, values[(size_t)(k0 + j) * kv_dim + lane + 64 * i], o[i]);
+  for (int k0 = k_lo; k0 < k_hi; k0 += 16 * NU) {
+    float x[NU][NE][4];
+#pragma unroll
+    for (int u = 0; u < NU; u++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const float* vp = values + (size_t)min(k0 + 16 * u + 4 * g4 + v, k_hi - 1) * kv_dim + l16;
+#pragma unroll
+        for (int e = 0; e < NE; e++) x[u][e][v] = vp[16 * e];
       }
-      m = m_new;
+    v4f s[NU];
+#pragma unroll
+    for (int u = 0; u < NU; u++) s[u] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int d = 0; d < ND; d++)
+#pragma unroll
+      for (int c = 0; c < 4; c++)
+#pragma unroll
+        for (int u = 0; u < NU; u++)
+          s[u] = __builtin_amdgcn_mfma_f32_16x16x4f32((&kr[u][d].x)[c], (&qr[d].x)[c], s[u], 0, 0, 0);
+    if (k0 + 16 * NU < k_hi) load_keys(k0 + 16 * NU);
+    float mt = -INFINITY, weight[NU][4];
+#pragma unroll
+    for (int u = 0; u < NU; u++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const uint32_t key = k0 + 16 * u + 4 * g4 + v;
+        weight[u][v] = (int)key < k_hi && key - see_lo < see_n ? 1.0f : 0.0f;
+        if (weight[u][v] == 0.0f) s[u][v] = -INFINITY;
+        mt = fmaxf(mt, s[u][v]);
+      }
+    const float m_new = fmaxf(m, rows4_max(mt) * sl), ref = m_new == -INFINITY ? 0.0f : m_new;
+    const float alpha = __builtin_amdgcn_exp2f(m - ref);
+    float ps = 0.0f;
+#pragma unroll
+    for (int u = 0; u < NU; u++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        s[u][v] = __builtin_amdgcn_exp2f(fmaf(s[u][v], sl, -ref));
+        ps += s[u][v];
+        if (s[u][v] == 0.0f) weight[u][v] *= 16384.0f;
+      }
+    l = l * alpha + rows4_sum(ps);
+    m = m_new;
+    if (!__any(l == l)) return;
+#pragma unroll
+    for (int e = 0; e < NE; e++) {
+      bool finite = true;
+#pragma unroll
+      for (int u = 0; u < NU; u++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) finite &= fabsf(x[u][e][v]) < INFINITY;
+      v4f d = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (__any(!finite)) {
+        v4f codes = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int u = 0; u < NU; u++)
+#pragma unroll
+          for (int v = 0; v < 4; v++) {
+            const float xv = x[u][e][v];
+            const float code = xv == INFINITY ? 1.0f : xv == -INFINITY ? 128.0f
+                               : xv != xv ? 129.0f : 0.0f;
+            codes = __builtin_amdgcn_mfma_f32_16x16x4f32(code, weight[u][v], codes, 0, 0, 0);
+            x[u][e][v] = code == 0.0f ? xv : 0.0f;
+          }
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const float minus = floorf(codes[v] * (1.0f / 128.0f));
+          const float up = codes[v] - 128.0f * minus > 0.0f ? INFINITY : 0.0f;
+          const float down = minus > 0.0f ? INFINITY : 0.0f;
+          d[v] = codes[v] >= 16384.0f ? NAN : up - down;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < NU; u++)
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+          d = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u][e][v], s[u][v], d, 0, 0, 0);
+#pragma unroll
+      for (int v = 0; v < 4; v++) o[e][v] = fmaf(o[e][v], alpha, d[v]);
     }
-    const float g = gate != nullptr ? 1.0f / (1.0f + expf(-gate[th])) : 1.0f;
-    float* w = splits > 1 ? ws + (th * splits + split) * (HD + 4) : nullptr;
-    for (int i = 0; i < ND; i++) {
-      if (w != nullptr) w[4 + lane + 64 * i] = o[i];
-      else out[th * HD + lane + 64 * i] = gate != nullptr ? (o[i] / l) * g : o[i] / l;
-    }
-    if (w != nullptr && lane < 2) w[lane] = lane == 0 ? m : l;
   }
 }
 
@@ -981,7 +1058,6 @@ attention_prefill_kernel(const float* __restrict__ q, const float* __restrict__ 
   constexpr int KT = T::KT, NS = KT / 16, NE = HD / 16;
   constexpr int QW = 4 / GW;                     // query blocks of a workgroup
   __shared__ __align__(16) uint8_t lds[T::kK + T::kV];
-  __shared__ int special[2];   // tile t (t % 2) holds an infinity or NaN
   uint8_t* Kp = lds;
   uint8_t* Vp = lds + T::kK;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1032,15 +1108,14 @@ attention_prefill_kernel(const float* __restrict__ q, const float* __restrict__ 
       }
     }
   };
-  auto store_tile = [&](int t) {
-    float rest = 0.0f;
+  auto store_tile = [&] {
     uint4 p[3];
     if (v_half) {
 #pragma unroll
       for (int d = 0; d < 4; d++) {
         const float x[8] = {(&raw[0].x)[d], (&raw[1].x)[d], (&raw[2].x)[d], (&raw[3].x)[d],
                             (&raw[4].x)[d], (&raw[5].x)[d], (&raw[6].x)[d], (&raw[7].x)[d]};
-        rest += split_pieces(x, p);
+        split_pieces(x, p);
         // Rows of four dims, 64 bytes, would meet in the same banks for
         // threads two apart: the row's place is turned by bits 3, 4 of the dim.
         const int slot = 4 * vd + (d ^ ((vd >> 1) & 3));
@@ -1054,13 +1129,12 @@ attention_prefill_kernel(const float* __restrict__ q, const float* __restrict__ 
         const int u = j * 128 + su, key = u / (HD / 8), g = u % (HD / 8);
         const float x[8] = {raw[2 * j].x,     raw[2 * j].y,     raw[2 * j].z,     raw[2 * j].w,
                             raw[2 * j + 1].x, raw[2 * j + 1].y, raw[2 * j + 1].z, raw[2 * j + 1].w};
-        rest += split_pieces(x, p);
+        split_pieces(x, p);
 #pragma unroll
         for (int i = 0; i < 3; i++)
           *(uint4*)(Kp + (i * (HD / 8) + g) * T::KS + key * 16) = p[i];
       }
     }
-    if (!(fabsf(rest) < INFINITY)) special[t & 1] = 1;
   };
 
   // B operand of S^T: the lane's query, dims 32 s + 8 g4 + 0..7, in pieces.
@@ -1077,16 +1151,11 @@ attention_prefill_kernel(const float* __restrict__ q, const float* __restrict__ 
   }
   load_tile(tile_lo);
   uint4 qf[HD / 32][3];
-  bool plain;   // an infinity or NaN was met: the wave's rows are formed anew
-  {
-    float rest = 0.0f;
 #pragma unroll
-    for (int s = 0; s < HD / 32; s++) {
-      const float4 a = qv[2 * s], b = qv[2 * s + 1];
-      const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-      rest += split_pieces(x, qf[s]);
-    }
-    plain = __any(!(fabsf(rest) < INFINITY));
+  for (int s = 0; s < HD / 32; s++) {
+    const float4 a = qv[2 * s], b = qv[2 * s + 1];
+    const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    split_pieces(x, qf[s]);
   }
   // The keys that the lane's query sees: see_lo .. see_lo + see_n - 1.
   const uint32_t see_lo = window > 0 ? max(0, qpos - window + 1) : 0;
@@ -1095,19 +1164,15 @@ attention_prefill_kernel(const float* __restrict__ q, const float* __restrict__ 
   v4f o[NE];
 #pragma unroll
   for (int e = 0; e < NE; e++) o[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-  if (tid < 2) special[tid] = 0;
 
   for (int t = tile_lo; t < tile_hi; t++) {
     __syncthreads();  // every wave is done with the previous tile
-    store_tile(t);
+    store_tile();
     __syncthreads();
     if (t + 1 < tile_hi) load_tile(t + 1);  // in flight during this tile's math
-    const bool tile_special = special[t & 1] != 0;
-    if (tid == 0) special[(t + 1) & 1] = 0;   // its last readers are past the barriers
     const int kt = kr.start + t * KT;
     const int q_hi = position + min(t0 + kPQ, n) - 1;   // the wave's last query's place
     if (t0 >= n || kt > q_hi) continue;                 // no query of the wave sees a key
-    plain |= tile_special;
 
     // Scores of keys kt + 16 u + 4 g4 + v.
     v4f s[NS];
@@ -1177,11 +1242,19 @@ attention_prefill_kernel(const float* __restrict__ q, const float* __restrict__ 
       for (int v = 0; v < 4; v++) o[e][v] = fmaf(o[e][v], alpha, d[v]);
     }
   }
-  if (plain) {
-    prefill_plain<HD>(q, keys + kvo, values + kvo, gate, out, ws, position, n, heads, head, kv_dim,
-                      window, sl, t0, kr.start + tile_lo * KT, min(kr.end, kr.start + tile_hi * KT),
-                      splits, split, lane);
-    return;
+  // NaN if a sum is (an infinity or NaN in Q or K, or a score that overflowed,
+  // makes l NaN), or if one is infinite.
+  float check = l_run - l_run;
+#pragma unroll
+  for (int e = 0; e < NE; e++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) check += o[e][v] - o[e][v];
+  if (__builtin_expect(__any(check != check), 0)) {
+    const int first = window > 0 ? max(0, position + t0 - window + 1) : 0;
+    prefill_special<HD>(q + ((size_t)min(tq, n - 1) * heads + head) * HD, keys + kvo,
+                        values + kvo, kv_dim, sl, max(first, kr.start + tile_lo * KT),
+                        min(min(kr.end, position + min(t0 + kPQ, n)), kr.start + tile_hi * KT),
+                        see_lo, see_n, lane, m_run, l_run, o);
   }
   // The lane's query, dims 16 e + 4 g4 + 0..3: 64 bytes of a row per store
   // and query.

@@ -175,6 +175,115 @@ def test_prefill_attention_special_values(gpu_ready, pos, n, hd):
             assert ok, (t, h, err)
 
 
+def special_prefill(rng, heads, kv, hd, pos, n):
+    """Inputs with an infinity or NaN of each kind, so placed that rows of
+    finite results remain: the oracle says which."""
+    q = rng.standard_normal((n, heads, hd)).astype(np.float32)
+    keys = rng.standard_normal((pos + n, kv, hd)).astype(np.float32)
+    values = rng.standard_normal((pos + n, kv, hd)).astype(np.float32)
+    at = lambda share: pos + int(n * share)
+    q[:, :, 5] = np.abs(q[:, :, 5]) + 0.1
+    q[n // 5, 0, 7] = np.nan
+    q[n // 4, 1, 7] = np.inf
+    keys[at(0.1), :, 5] = -np.inf        # a score of -inf: counts for nothing
+    keys[at(0.95), 0, 8] = np.nan
+    values[at(0.1), 0, 1] = -3.4e38      # of a key that counts for nothing
+    values[at(0.3), 0, 9] = np.inf
+    values[at(0.5), -1, 10] = -np.inf
+    values[at(0.6), -1, 10] = np.inf     # both: NaN
+    values[at(0.7), :, 11] = np.nan
+    values[at(0.8), -1, 12] = 3.39e38    # no infinity, but rounds to one as bf16
+    return q, keys, values
+
+
+# Windows (a key leaves a query's view again), gates, whole key ranges (the
+# first of each three) and split ones, a ragged last wave.
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("heads,kv,pos,n,window,gated", [
+    (2, 1, 0, 45, 0, True), (4, 2, 700, 64, 0, True), (8, 2, 300, 77, 0, False),
+    (2, 2, 20, 50, 16, False), (4, 1, 500, 90, 40, True), (4, 4, 1000, 33, 300, False)])
+def test_prefill_attention_special_values_window_gate(gpu_ready, orc, heads, kv, pos, n, window,
+                                                      gated, hd):
+    rng = np.random.default_rng(heads + pos + n + window)
+    q, keys, values = special_prefill(rng, heads, kv, hd, pos, n)
+    gate = rng.standard_normal(n * heads).astype(np.float32) if gated else None
+    print(f"special prefill {heads}/{kv} hd={hd} {n} after {pos} window={window}", flush=True)
+    out = torch.full((n * heads * hd,), 7.0, device="cuda")
+    D.attention(dev(q), dev(keys), dev(values), dev(gate) if gated else None, out, pos, n, heads,
+                kv, hd, window)
+    got = host(out).reshape(n, heads, hd)
+    want = orc.attention(q, keys, values, gate, pos, n, heads, kv, hd, window).reshape(got.shape)
+    finite = np.isfinite(want)
+    assert 0.3 < finite.mean() < 0.999
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    got, want = got[finite], want[finite]
+    # The oracle's terms are float32 rounded once; a huge value leaves an
+    # absolute error of its own size times 2^-22 in its row.
+    small = np.abs(want) < 1e6
+    ok, err = close(got[small], want[small])
+    assert ok, err
+    assert np.all(np.abs(got - want)[~small] <= 1e-5 * np.abs(want[~small]))
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("pos,n", [(0, 45), (600, 64)])
+def test_prefill_attention_special_values_overflow(gpu_ready, orc, pos, n, hd):
+    """Finite operands whose product is past the largest float: a score of
+    -inf, which counts for nothing. (1.005e30 is rounded up to bf16, so its
+    pieces have both signs and so have their products' infinities.)"""
+    heads, kv = 4, 2
+    rng = np.random.default_rng(pos + n)
+    q = rng.standard_normal((n, heads, hd)).astype(np.float32)
+    keys = rng.standard_normal((pos + n, kv, hd)).astype(np.float32)
+    values = rng.standard_normal((pos + n, kv, hd)).astype(np.float32)
+    q[:, :, 6] = 1.005e30
+    keys[:, :, 6] *= 1e-30
+    keys[pos + 1, :, 6] = -1.005e30
+    out = torch.full((n * heads * hd,), 7.0, device="cuda")
+    D.attention(dev(q), dev(keys), dev(values), None, out, pos, n, heads, kv, hd)
+    want = orc.attention(q, keys, values, None, pos, n, heads, kv, hd, 0)
+    assert np.isfinite(want).all()
+    ok, err = close(host(out), want)
+    assert ok, err
+
+
+def test_prefill_attention_special_values_cost(gpu_ready):
+    """Infinities and NaN cost a prefill a second walk over the keys and no
+    more: measured at 2.2 times the finite call here, with a bar of eight (a
+    query at a time in plain loads took fifty)."""
+    heads, kv, hd, pos, n = 16, 8, 128, 1000, 512
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q = torch.randn(n, heads, hd, device="cuda", generator=g)
+    keys = torch.randn(pos + n, kv, hd, device="cuda", generator=g)
+    values = torch.randn(pos + n, kv, hd, device="cuda", generator=g)
+    out = torch.empty(n, heads, hd, device="cuda")
+
+    def ms(q, keys, values):
+        best = 1e9
+        for _ in range(4):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(5):
+                D.attention(q, keys, values, None, out, pos, n, heads, kv, hd)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    finite = ms(q, keys, values)
+    for what, at in (("all nan", None), ("inf value", 700), ("nan key", 700)):
+        t = [x.clone() for x in (q, keys, values)]
+        if at is None:
+            for x in t:
+                x.fill_(float("nan"))
+        else:
+            t[2 if what == "inf value" else 1][at, :, 3] = float(what[:3])
+        took = ms(*t)
+        print(f"{what}: {took / 5 * 1e3:.0f} us, finite {finite / 5 * 1e3:.0f}", flush=True)
+        assert took < 8 * finite, (what, took, finite)
+
+
 def test_attention_limits(gpu_ready):
     lib = _lib.load()
     assert lib.dnx_attention_max_keys(128) >= 15000
