@@ -813,8 +813,12 @@ attention_combine_kernel(const float* __restrict__ ws, const float* __restrict__
 //   operand as they are if k slot j of lane group g stands for key 4 g + j
 //   (j < 4) or 16 + 4 g + j - 4; V^T is staged in that order.
 // A tile's products start from zero and join the running sums in one
-// multiply-add, so a long run rounds once a tile (64 bits say 3.9e-7 after
-// 4000 keys where sums carried through the MFMAs had 9.5e-7).
+// multiply-add, so a long run rounds once a tile; within a tile the products
+// of first pieces have a sum of their own (mfma_pieces). Error against 64
+// bits, relative 2-norm, with the float32 MFMAs -> so: 64 tokens after 256
+// (16 / 8 heads, hd 128) 2.8e-7 -> 1.7e-7 (3.0e-7 with all six products in one
+// sum), 512 from 0 (32 / 8) 2.5e-7 -> 1.2e-7, 1000 after 1000 (16 / 8) 6.0e-7
+// -> 2.1e-7, 8 after 4000 (8 / 2, hd 64) 3.0e-7 -> 2.3e-7.
 // A wave whose queries see no key of a tile skips it; only tiles at the edge
 // of the causal or window range are masked.
 //
@@ -912,14 +916,20 @@ DNX_DEV void split_pieces(const float* x, uint4* p) {
   for (int i = 0; i < 3; i++) p[i] = make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]);
 }
 
-// acc += A B over the six piece products, the smallest first.
-DNX_DEV v4f mfma_pieces(const uint4* a, const uint4* b, v4f acc) {
-  constexpr int kA[6] = {2, 1, 0, 1, 0, 0}, kB[6] = {0, 1, 2, 0, 1, 0};
-#pragma unroll
-  for (int i = 0; i < 6; i++)
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, a[kA[i]]),
-                                                  __builtin_bit_cast(bf8, b[kB[i]]), acc, 0, 0, 0);
-  return acc;
+// big += A0 B0 and low += the five other piece products, the smallest first.
+// Each product rounds its sum: low rounds at 2^-8 of big or less, where all
+// six in one sum rounded it six times a step at its full size.
+DNX_DEV void mfma_pieces(const uint4* a, const uint4* b, v4f& big, v4f& low) {
+  auto product = [&](int i, int j, v4f acc) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, a[i]),
+                                                   __builtin_bit_cast(bf8, b[j]), acc, 0, 0, 0);
+  };
+  big = product(0, 0, big);
+  low = product(2, 0, low);
+  low = product(1, 1, low);
+  low = product(0, 2, low);
+  low = product(1, 0, low);
+  low = product(0, 1, low);
 }
 
 // The sums (m, l, o) of a wave's 16 queries over keys k_lo .. k_hi - 1 where
@@ -1175,9 +1185,9 @@ attention_prefill_kernel(const float* __restrict__ q, const float* __restrict__ 
     if (t0 >= n || kt > q_hi) continue;                 // no query of the wave sees a key
 
     // Scores of keys kt + 16 u + 4 g4 + v.
-    v4f s[NS];
+    v4f s[NS], low[NS];
 #pragma unroll
-    for (int u = 0; u < NS; u++) s[u] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int u = 0; u < NS; u++) s[u] = low[u] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int d = 0; d < HD / 32; d++) {
 #pragma unroll
@@ -1186,9 +1196,11 @@ attention_prefill_kernel(const float* __restrict__ q, const float* __restrict__ 
 #pragma unroll
         for (int i = 0; i < 3; i++)
           kf[i] = *(const uint4*)(Kp + (i * (HD / 8) + 4 * d + g4) * T::KS + (16 * u + l16) * 16);
-        s[u] = mfma_pieces(kf, qf[d], s[u]);
+        mfma_pieces(kf, qf[d], s[u], low[u]);
       }
     }
+#pragma unroll
+    for (int u = 0; u < NS; u++) s[u] += low[u];
     const bool edge = kt + KT > position + t0 + 1 || kt + KT > kr.end ||
                       (window > 0 && kt <= q_hi - window);
     float mt = -INFINITY;
@@ -1228,7 +1240,7 @@ attention_prefill_kernel(const float* __restrict__ q, const float* __restrict__ 
     // multiply-add (with the rescale): one rounding a tile of a long run.
 #pragma unroll
     for (int e = 0; e < NE; e++) {
-      v4f d = {0.0f, 0.0f, 0.0f, 0.0f};
+      v4f d = {0.0f, 0.0f, 0.0f, 0.0f}, low = d;
 #pragma unroll
       for (int h = 0; h < KT / 32; h++) {
         uint4 vf[3];
@@ -1236,8 +1248,9 @@ attention_prefill_kernel(const float* __restrict__ q, const float* __restrict__ 
 #pragma unroll
         for (int i = 0; i < 3; i++)
           vf[i] = *(const uint4*)(Vp + (i * (KT / 8) + 4 * h + g4) * T::VS + slot * 16);
-        d = mfma_pieces(vf, pf[h], d);
+        mfma_pieces(vf, pf[h], d, low);
       }
+      d += low;
 #pragma unroll
       for (int v = 0; v < 4; v++) o[e][v] = fmaf(o[e][v], alpha, d[v]);
     }

@@ -267,6 +267,7 @@ def test_prepacked_gemm_equals_engine_layout(gpu_ready, orc, rows, cols, n):
     (2081, 64, 400),     # 64 (Q8: 32, two workgroups a CU)
     (4227, 96, 513),     # 96
     (6146, 96, 512),     # 128
+    (6146, 512, 512),    # 128, two stages of K (Q8: four)
 ])
 def test_prepacked_gemm_tile_edges(gpu_ready, q8, rows, cols, n):
     """Every workgroup shape: an output's bits do not depend on the rows and
@@ -300,6 +301,32 @@ def test_prepacked_gemm_tile_edges(gpu_ready, q8, rows, cols, n):
         for t0, t1 in [(0, 7), (120, 140), (n - 1, n)]:
             part = product(r0, r1, t0, t1)
             assert np.array_equal(bits(part), bits(whole[t0:t1, r0:r1])), (r0, r1, t0, t1)
+
+
+@pytest.mark.parametrize("q8", [False, True])
+@pytest.mark.parametrize("rows,cols,n", [(6146, 1056, 512), (8190, 1312, 490)])
+def test_prepacked_gemm_128_rows_many_stages(gpu_ready, orc, q8, rows, cols, n):
+    """128-row tiles over 5 and 6 stages of K (Q8: 9 and 11), so that both weight
+    buffers are filled again while the other is multiplied; K is not split.
+    Q4 gives the bits of the kernel on the engine's own layout; both stay
+    within the products' bar."""
+    rng = np.random.default_rng(rows + cols)
+    qs, sc = (synth.q8_weights if q8 else synth.q4_weights)(rng, rows, cols)
+    xs = synth.activations(rng, n, cols)
+    panel = torch.empty(D.f6_panel_bytes(n, cols), dtype=torch.uint8, device="cuda")
+    D.quantize_q8_f6panel(dev(xs), panel, n, cols)
+    packed = torch.empty((D.q8_f6pack_bytes if q8 else D.q4_f6pack_bytes)(rows, cols),
+                         dtype=torch.uint8, device="cuda")
+    (D.pack_q8_f6 if q8 else D.pack_q4_f6)(dev(qs), dev(sc), packed, rows, cols)
+    y = torch.full((n * rows,), float("nan"), device="cuda")
+    (D.gemm_q8_f6p if q8 else D.gemm_q4_f6p)(packed, panel, y, rows, cols, n)
+    got = host(y).reshape(n, rows)
+    if not q8:
+        D.gemm_q4_f6(dev(qs), dev(sc), panel, y, rows, cols, n)
+        assert np.array_equal(bits(got), bits(host(y).reshape(n, rows)))
+    ref = (orc.gemm_q8 if q8 else orc.gemm_q4)(qs, sc, xs, n, threads=8, mode=1)
+    ok, worst_rel, worst_abs = within_tolerance(got, ref)
+    assert ok, (worst_rel, worst_abs)
 
 
 @pytest.mark.parametrize("kernel", ["f6", "f6p", "f6s", "i8p", "i8p_wide", "i8p_split"])

@@ -56,3 +56,26 @@ def test_gelu_bit_exact_over_magnitudes(gpu_ready, orc, low, high):
     nan = np.isnan(want)
     assert np.array_equal(np.isnan(got), nan)
     assert np.array_equal(bits(got[~nan]), bits(want[~nan]))
+
+
+def test_gelu_every_float(gpu_ready):
+    """All 2^32 floats against the formula as it is written, two IEEE
+    divisions and the device's exp, one operation at a time in float64: the
+    kernel's product with a residual step and its Newton steps give the same
+    float for every input."""
+    sqrt2 = torch.tensor(1.4142135623730951, dtype=torch.float64, device="cuda")
+    step = 1 << 24
+    for first in range(-(1 << 31), 1 << 31, step):
+        x = torch.arange(first, first + step, dtype=torch.int32, device="cuda").view(torch.float32)
+        v = x.double()
+        z = v.abs() / sqrt2          # (a divisor that is a number would be a product)
+        t = torch.ones_like(z) / (1 + 0.3275911 * z)
+        poly = ((((1.061405429 * t - 1.453152027) * t + 1.421413741) * t - 0.284496736) * t
+                + 0.254829592) * t
+        erf = 1 - poly * torch.exp(-z * z)
+        want = (0.5 * v * (1 + torch.where(v < 0, -erf, erf))).float()
+        D.gelu(x)
+        nan = torch.isnan(want)
+        assert torch.equal(torch.isnan(x), nan), hex(first)
+        differ = (x.view(torch.int32) != want.view(torch.int32)) & ~nan
+        assert int(differ.sum()) == 0, (hex(first), int(differ.sum()))

@@ -175,6 +175,35 @@ def test_prefill_attention_special_values(gpu_ready, pos, n, hd):
             assert ok, (t, h, err)
 
 
+# The bar: the error of attention on the float32 matrix cores on these inputs.
+@pytest.mark.parametrize("heads,kv,hd,pos,n,bar", [
+    (16, 8, 128, 256, 64, 2.89e-7), (8, 2, 128, 1785, 20, 3.06e-7), (32, 8, 128, 0, 256, 2.03e-7),
+    (8, 8, 64, 500, 37, 2.55e-7), (8, 2, 64, 4000, 8, 2.89e-7)])
+def test_prefill_attention_precision(gpu_ready, heads, kv, hd, pos, n, bar):
+    """No further from 64 bits than float32 products are. A result is rounded
+    about twelve times at its own size (the first pieces' products, the joining
+    of the tiles, the weights' sum, a division): a random walk of 2^-24 /
+    sqrt(3) each is 1.2e-7, and the scores' rounding, which the exponential
+    carries into the weights, adds about as much (1.1 to 2.2e-7 measured)."""
+    rng = np.random.default_rng(heads + hd + pos + n)
+    q = rng.standard_normal((n, heads, hd)).astype(np.float32)
+    keys = rng.standard_normal((pos + n, kv, hd)).astype(np.float32)
+    values = rng.standard_normal((pos + n, kv, hd)).astype(np.float32)
+    out = torch.zeros(n * heads * hd, device="cuda")
+    D.attention(dev(q), dev(keys), dev(values), None, out, pos, n, heads, kv, hd)
+    got = host(out).reshape(n, heads, hd)
+    hidden = np.arange(pos + n)[None] > pos + np.arange(n)[:, None]
+    want = np.empty(got.shape)
+    for h in range(heads):
+        s = q[:, h].astype(np.float64) @ keys[:, h // (heads // kv)].T.astype(np.float64)
+        s = np.where(hidden, -np.inf, s / np.sqrt(hd))
+        p = np.exp(s - s.max(1, keepdims=True))
+        want[:, h] = p / p.sum(1, keepdims=True) @ values[:, h // (heads // kv)].astype(np.float64)
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
+    print(f"{heads}/{kv} hd={hd} {n} after {pos}: {err:.2e}", flush=True)
+    assert err < bar
+
+
 def special_prefill(rng, heads, kv, hd, pos, n):
     """Inputs with an infinity or NaN of each kind, so placed that rows of
     finite results remain: the oracle says which."""
