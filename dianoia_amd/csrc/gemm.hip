@@ -21,6 +21,7 @@
 
 #include "common.h"
 #include "dnx_kernels.h"
+#include "gemm_route.h"
 
 using namespace dnx;
 
@@ -308,21 +309,11 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(GemmParams p) {
 // wave order (deterministic), with no split-K pass. Rows past the matrix
 // and tokens past n load zeros (bounded buffer loads) and are not stored;
 // blocks past a wave's last load zeros and add exact zeros.
-constexpr int kSkinnyRows = 16;
 constexpr int kSkinnyBlocks = 16;       // blocks per wave: K <= 2048
 constexpr int kSkinnyFar = 0x7fffff00;  // a buffer offset past every operand
 
 typedef int v2i_t __attribute__((ext_vector_type(2)));
 typedef int v4i_t __attribute__((ext_vector_type(4)));
-
-// LDS of the skinny kernel: padded weight rows, weight scales (fp32), x
-// scales [block][token], and waves 1..3's sums.
-size_t skinny_row_bytes(bool q4, int cols) { return (size_t)(q4 ? cols / 2 : cols) + 16; }
-size_t skinny_lds(bool q4, int cols, int mt) {
-  const int blocks = cols / kBlock;
-  return kSkinnyRows * skinny_row_bytes(q4, cols) + (size_t)kSkinnyRows * blocks * 4 +
-         (size_t)blocks * 16 * mt * 4 + (size_t)3 * mt * 4 * 64 * 4;
-}
 
 template <bool kQ4, int MT>
 __global__ void __launch_bounds__(kThreads) skinny_kernel(GemmParams p) {
@@ -468,15 +459,6 @@ __global__ void __launch_bounds__(kThreads) skinny_kernel(GemmParams p) {
     }
 }
 
-// Whether the skinny kernel takes this shape: n <= 16, K <= 2048 (16
-// blocks per wave, 8 row pieces per thread) and the LDS within 64 KB. With
-// more tokens it lost to the split-K tile kernel on 6144 x 2048 Q4 (n = 32:
-// 13.7 against 11.8 us; n = 16: 9.7 against 10.2; n = 8: 8.5 against 9.4).
-bool skinny_fits(bool q4, int64_t cols, int64_t n) {
-  if (n > 16 || cols > 2048 || cols % 16 != 0) return false;
-  return skinny_lds(q4, (int)cols, 1) <= 64 * 1024;
-}
-
 template <bool kQ4, int MT>
 int launch_skinny(const GemmParams& p, hipStream_t stream) {
   const size_t lds = skinny_lds(kQ4, p.cols, MT);
@@ -487,7 +469,8 @@ int launch_skinny(const GemmParams& p, hipStream_t stream) {
 
 // ---------------------------------------------------------- chunk (n > 16)
 
-// A prompt chunk (the decoder's 5..64 tokens) in one launch over the whole K:
+// A prompt chunk (17 tokens or more, up to 256 workgroups) in one launch over
+// the whole K:
 // a workgroup owns 32 weight rows and G * 32 tokens, and its 8 waves share K
 // in units of 4 blocks (wave w: units w, w + 8, ...), so a wave's loads of a
 // row use its whole 128-byte lines. Both operands come straight from memory
@@ -642,35 +625,6 @@ __global__ void __launch_bounds__(kChunkThreads) chunk_kernel(GemmParams p) {
     }
 }
 
-// Token groups per workgroup of the chunk kernel for a shape, 0 where the
-// tile kernel is the faster (graph-timed with the quantizer, us, tile kernel
-// against this):
-// * one round of 256 workgroups, or the second round's tail costs more than
-//   the tile kernel's reduce (3072 x 1024 at 200 tokens: 14.6 against 14.4,
-//   6144 x 1024 at 200 14.9 against 20.0);
-// * K <= 1024 (a wave's blocks all requested at once): Q8 3072 x 1024 at 33 /
-//   64 / 128 tokens 9.2 / 10.8 / 12.2 against 7.2 / 7.3 / 9.0, Q4 9.2 / 10.9 /
-//   12.0 against 7.8 / 7.9 / 9.7, 512 x 512 at 17..256 7.7..8.5 against 5.7..6.3;
-// * K <= 2048 (two units a wave) where the launch fills the chip enough: 2048
-//   x 2048 Q8 at 64 / 128 12.8 / 13.7 against 10.2 / 10.4, Q4 12.5 / 13.6
-//   against 11.4 / 11.9; with 64 workgroups or fewer (512 x 2048 Q8 at 64: 9.0
-//   against 9.9), and below 64 tokens of Q4 (2048 x 2048 at 33: 10.1 against
-//   11.3), the tile kernel's K split wins;
-// * longer K: each unit adds a memory round trip (1024 x 3072 at 64: 11.7
-//   against 12.9).
-// Up to 16 tokens the skinny kernel's sums are closer to 64 bits (7.2e-8
-// against 8.4e-8 at K = 1024) and it keeps them.
-int chunk_groups(bool q4, int64_t rows, int64_t cols, int64_t n) {
-  const int64_t blocks = cols / kBlock, row_groups = (rows + 31) / 32;
-  if (n <= 16 || blocks > 64) return 0;
-  for (int g = 1; g <= 2; g++) {
-    const int64_t wgs = row_groups * ((n + 32 * g - 1) / (32 * g));
-    if (wgs > 256) continue;
-    return blocks <= 32 || (wgs > 64 && (!q4 || n >= 64)) ? g : 0;
-  }
-  return 0;
-}
-
 template <bool kQ4, int G>
 int launch_chunk(const GemmParams& p, hipStream_t stream) {
   const dim3 grid((unsigned)((p.rows + 31) / 32), (unsigned)((p.n + G * 32 - 1) / (G * 32)));
@@ -710,29 +664,13 @@ float* split_workspace(size_t bytes) {
   return gSplitWs;
 }
 
-template <bool kQ4, int BM, int BN, int WM, int KB>
+template <bool kQ4, int BM, int BN, int WM>
 int launch_tile(GemmParams p, hipStream_t stream) {
+  constexpr int KB = kTileBlocks;
   const unsigned gx = (unsigned)((p.rows + BN - 1) / BN), gy = (unsigned)((p.n + BM - 1) / BM);
   const int stages = (p.cols / kBlock + KB - 1) / KB;
-  // Split K when the tiles alone would leave CUs idle (small n): enough
-  // splits for about 512 workgroups, each with at least one stage. Between
-  // one and three workgroups per CU (the resident count of the 64 x 64
-  // tiles) a long K (32+ stages) is split too, into runs of at least 8
-  // stages, so that the slots fill: the vision fc2 (1152 x 4320 at 1024
-  // tokens, 288 tiles) ran one or two workgroups per CU over all 34 stages
-  // (47.9 -> 42.6 us with 3 splits). A shorter K loses more to the partials'
-  // round trip than it gains (6144 x 2048 at 256 tokens: 24 -> 27 us).
-  int splits = 1;
-  const int64_t tiles = (int64_t)gx * gy;
-  if (tiles < 256 && stages > 1) {
-    splits = (int)((512 + tiles - 1) / tiles);
-    if (splits > stages) splits = stages;
-  } else if (tiles < 768 && stages >= 32) {
-    splits = (int)((768 + tiles - 1) / tiles);
-    if (splits > stages / 8) splits = stages / 8;
-  }
-  p.split_stages = (stages + splits - 1) / splits;
-  splits = (stages + p.split_stages - 1) / p.split_stages;
+  p.split_stages = tile_split_stages((int64_t)gx * gy, stages);
+  const int splits = (stages + p.split_stages - 1) / p.split_stages;
   p.part = nullptr;
   const int64_t count = (int64_t)p.n * p.rows;
   if (splits > 1) {
@@ -759,18 +697,13 @@ int launch_gemm(const void* qs, const void* scales, const int8_t* xq, const floa
   if (rows * (kQ4 ? cols / 2 : cols) >= (1ll << 31) || n * cols >= (1ll << 31)) return DNX_EINVAL;
   if (((uintptr_t)qs & 15) || ((uintptr_t)xq & 15) || (cols % 16)) return DNX_EINVAL;
   GemmParams p{qs, scales, xq, xsc, y, (int)rows, (int)cols, (int)n, 0, nullptr};
-  // Up to 16 tokens and K <= 2048: the skinny kernel (every load at the
-  // start, K shared by a workgroup's waves, no split-K pass);
-  // 32 tokens: one wave row of 32 x 32 tiles (4 waves across N); else
-  // 64 x 64 tiles (2 x 2 waves), which keep ~3 workgroups per CU resident
-  // at prefill sizes.
-  if (skinny_fits(kQ4, cols, n)) return launch_skinny<kQ4, 1>(p, stream);
-  switch (chunk_groups(kQ4, rows, cols, n)) {
-    case 1: return launch_chunk<kQ4, 1>(p, stream);
-    case 2: return launch_chunk<kQ4, 2>(p, stream);
+  switch (gemm_kernel_for(kQ4, rows, cols, n)) {
+    case GemmKernel::kSkinny: return launch_skinny<kQ4, 1>(p, stream);
+    case GemmKernel::kChunk1: return launch_chunk<kQ4, 1>(p, stream);
+    case GemmKernel::kChunk2: return launch_chunk<kQ4, 2>(p, stream);
+    case GemmKernel::kTile32: return launch_tile<kQ4, 32, 128, 1>(p, stream);
+    default: return launch_tile<kQ4, 64, 64, 2>(p, stream);
   }
-  if (n <= 32) return launch_tile<kQ4, 32, 128, 1, 4>(p, stream);
-  return launch_tile<kQ4, 64, 64, 2, 4>(p, stream);
 }
 
 }  // namespace
