@@ -204,12 +204,12 @@ int dnx_gemm_q4_float(const uint8_t* qs, const uint16_t* scales, const float* x,
 // (xq int8 [n][cols], xsc fp32 [n][cols/32], e.g. by dnx_quantize_q8):
 // the per-32-block int32 dots are exact, the per-block scaling is fp32
 // (within 1e-4 relative of the CPU kernels, not bit-identical; the same
-// inputs always give the same bits). Up to 16 tokens, and for the chunks
-// that fit one round of workgroups, K <= 2048 runs in one launch; else when n
-// is small (fewer than 256 output tiles) K is split across workgroups and a second kernel sums the partials
-// in a fixed order; their workspace is the library's own, allocated on the
-// first such call at a larger shape (so that call must not be captured into
-// a graph).
+// inputs always give the same bits). One launch, and no memory but the
+// arguments': n <= 16 with K <= 2048, and K <= 1024 where
+// ceil(rows / 32) * ceil(n / 64) <= 256. Any other call may split K across
+// workgroups; a second kernel then sums the partials in a fixed order, in a
+// workspace of the library's own, which the first such call at a larger shape
+// allocates (so that call must not be captured into a graph).
 int dnx_gemm_q8(const int8_t* qs, const float* scales, const int8_t* xq, const float* xsc,
                 float* y, int64_t rows, int64_t cols, int64_t n, dnx_stream_t stream);
 int dnx_gemm_q4(const uint8_t* qs, const uint16_t* scales, const int8_t* xq, const float* xsc,
@@ -467,8 +467,10 @@ int dnx_short_conv(const float* bcx, const float* weight, float* history, float*
 // [n][heads][hd], gate [n][heads] or null (ungated); window 0: every earlier
 // position, else the last `window`. hd a multiple of 4 dividing 256; q and
 // keys 16-byte aligned. 8+ tokens at hd 64 or 128 with a 16-byte aligned
-// out run on the bf16 matrix cores, each operand as three exact pieces; decode-shaped calls (fewer than 256
-// head-token pairs, more than 256 keys) split the keys over workgroups.
+// out run on the bf16 matrix cores, each operand as three pieces, whose sum it
+// is exactly down to 2^-110 (2e-7 of it is lost at 2^-112, 2e-3 at 2^-125);
+// decode-shaped calls (fewer than 256 head-token pairs, more than 256 keys)
+// split the keys over workgroups.
 // Both may add a combine pass over a library-owned workspace grown on
 // demand: a first call at a larger shape allocates (not inside a graph
 // capture), and calls that overlap (other streams, other threads) must not

@@ -67,3 +67,26 @@ def test_chunk_lines(route):
                         ((0, 1024, 2080, 64), "tile64"), ((0, 512, 160, 17), "chunk1"),
                         ((1, 4096, 2080, 8), "tile32"), ((1, 4096, 2080, 17), "tile32")]:
         assert route([shape])[0][0] == want, shape
+
+
+def test_calls_that_allocate_nothing(route):
+    """dnx_kernels.h names the calls that take no memory of the library's own,
+    so that a caller may capture them at once: none of them splits K, and the
+    sentence names no more than that."""
+    sizes = [1, 31, 32, 33, 512, 2048, 3072, 8192, 8193, 20000, 151936]
+    shapes = [(q4, rows, cols, n) for q4 in (0, 1) for rows in sizes
+              for cols in (32, 64, 128, 160, 512, 992, 1024, 1056, 2048, 2080, 4096)
+              for n in (1, 5, 16, 17, 32, 33, 63, 64, 65, 128, 200, 512, 1024)]
+    named = 0
+    for (q4, rows, cols, n), (kernel, splits) in zip(shapes, route(shapes)):
+        if (n <= 16 and cols <= 2048) or (cols <= 1024 and -(-rows // 32) * -(-n // 64) <= 256):
+            named += 1
+            assert splits == 1, (q4, rows, cols, n, kernel)
+    assert named > 800
+    header = open(os.path.join(CSRC, "..", "..", "include", "dnx_kernels.h")).read()
+    header = " ".join(header.replace("//", " ").split())
+    assert ("n <= 16 with K <= 2048, and K <= 1024 where ceil(rows / 32) * ceil(n / 64) <= 256. "
+            "Any other call may split K") in header
+    # Two that a line at K <= 2048 alone would name: they split K.
+    for shape in ((0, 512, 2048, 64), (1, 2048, 2048, 33)):
+        assert route([shape])[0][1] > 1
