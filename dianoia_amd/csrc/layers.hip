@@ -794,10 +794,11 @@ attention_combine_kernel(const float* __restrict__ ws, const float* __restrict__
 }
 
 // Attention of many tokens (prefill) on the bf16 matrix cores, float32 in and
-// out. Every float32 operand is the exact sum of three bf16 pieces (8
-// significant bits each); of the nine piece products of a q.k or p.v term the
-// six with i + j <= 2 are formed, the others lie below 2^-23 of the term, and
-// the sums are float32. Six bf16 MFMAs cost less than half of the float32
+// out. A float32 operand of 2^-110 or more is the exact sum of three bf16
+// pieces (8 significant bits each; below that the last piece is a bf16
+// subnormal or lost: 2e-7 of the operand at 2^-112, 2e-3 at 2^-125); of the
+// nine piece products of a q.k or p.v term the six with i + j <= 2 are formed,
+// the others lie below 2^-26 of the term, and the sums are float32. Six bf16 MFMAs cost less than half of the float32
 // ones they replace (v_mfma_f32_16x16x4f32: 32 multiply-adds a clock and
 // SIMD, 16x16x32_bf16: 512).
 //
@@ -850,9 +851,9 @@ constexpr int kPQ = 16;   // queries per wave
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
-template <int HD>
+template <int HD, int KT_>
 struct PrefillTile {
-  static constexpr int KT = 4096 / HD;          // keys per tile: 32 or 64
+  static constexpr int KT = KT_;                // keys per tile: 32 or 64
   static constexpr int KS = KT * 16 + 16;       // K: one 8-dim group of all keys, + pad
   static constexpr int VS = HD * 16;            // V^T: 8 keys of all dims
   static constexpr int kK = 3 * (HD / 8) * KS;  // [piece][dim group][key][16 B]
@@ -1057,14 +1058,14 @@ DNX_DEV void prefill_special(const float* qp, const float* keys, const float* va
   }
 }
 
-template <int HD, int GW>
+template <int HD, int GW, int KT_>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 3)))
 attention_prefill_kernel(const float* __restrict__ q, const float* __restrict__ keys,
                          const float* __restrict__ values, const float* __restrict__ gate,
                          float* __restrict__ out, float* __restrict__ ws, int position, int n,
                          int heads, int kv_dim, int group, int window, float scale, int splits,
                          int tiles_per_split) {
-  using T = PrefillTile<HD>;
+  using T = PrefillTile<HD, KT_>;
   constexpr int KT = T::KT, NS = KT / 16, NE = HD / 16;
   constexpr int QW = 4 / GW;                     // query blocks of a workgroup
   __shared__ __align__(16) uint8_t lds[T::kK + T::kV];
@@ -1088,15 +1089,18 @@ attention_prefill_kernel(const float* __restrict__ q, const float* __restrict__ 
   const size_t kvo = (size_t)(blockIdx.x * GW / group) * HD;
   const float sl = scale * 1.44269504088896341f;   // scores in units of log2
 
-  // Staging: the first half of the workgroup carries V (thread: 4 dims of the
-  // 8 keys of a key group), the second K (thread: 4 times 8 dims of a key).
+  // Staging: the first half of the workgroup carries V (thread: NV dims of the
+  // 8 keys of a key group), the second K (thread: NV times 8 dims of a key).
+  constexpr int NV = KT * HD / 1024;             // 4, or 2 where KT * HD is 2048
   const bool v_half = wave < 2;
   const int su = tid & 127;
-  const int vd = su % (HD / 4), vg = su / (HD / 4);   // V: dims 4 vd.., key group vg
-  float4 raw[8];
+  const int vd = su % (HD / NV), vg = su / (HD / NV);   // V: dims NV vd.., key group vg
+  // As loaded, whole vectors: taken apart here they would be waited for where
+  // they are loaded (1000 tokens after 1000: 97 -> 114 us).
+  float4 raw[2 * NV];
   // A resource per row of a thread's eight loads, so that one offset serves
   // them all; rows past the keys read zeros.
-  const int v_off = (32 * (vg >> 2) + 4 * (vg & 3)) * kv_dim * 4 + vd * 16;
+  const int v_off = (32 * (vg >> 2) + 4 * (vg & 3)) * kv_dim * 4 + vd * NV * 4;
   const int k_off = su / (HD / 8) * kv_dim * 4 + su % (HD / 8) * 32;
   auto load_tile = [&](int t) {
     const int kt = kr.start + t * KT, rows = min(KT, kr.end - kt);
@@ -1107,11 +1111,19 @@ attention_prefill_kernel(const float* __restrict__ q, const float* __restrict__ 
     };
     if (v_half) {
 #pragma unroll
-      for (int j = 0; j < 8; j++)
-        raw[j] = buffer_load_f4(row(values, 16 * (j >> 2) + (j & 3)), v_off);
+      for (int j = 0; j < 8; j++) {
+        const i32x4 r = row(values, 16 * (j >> 2) + (j & 3));
+        if constexpr (NV == 4) {
+          raw[j] = buffer_load_f4(r, v_off);
+        } else {
+          const i32x2 x = dnx_raw_buffer_load_v2i32(r, v_off, 0, 0);
+          (&raw[j >> 1].x)[2 * (j & 1)] = __int_as_float(x.x);
+          (&raw[j >> 1].x)[2 * (j & 1) + 1] = __int_as_float(x.y);
+        }
+      }
     } else {
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
+      for (int j = 0; j < NV; j++) {
         const i32x4 r = row(keys, j * (128 / (HD / 8)));
         raw[2 * j] = buffer_load_f4(r, k_off);
         raw[2 * j + 1] = buffer_load_f4(r, k_off + 16);
@@ -1122,23 +1134,24 @@ attention_prefill_kernel(const float* __restrict__ q, const float* __restrict__ 
     uint4 p[3];
     if (v_half) {
 #pragma unroll
-      for (int d = 0; d < 4; d++) {
-        const float x[8] = {(&raw[0].x)[d], (&raw[1].x)[d], (&raw[2].x)[d], (&raw[3].x)[d],
-                            (&raw[4].x)[d], (&raw[5].x)[d], (&raw[6].x)[d], (&raw[7].x)[d]};
+      for (int d = 0; d < NV; d++) {
+        float x[8];   // dim d of the eight keys
+#pragma unroll
+        for (int j = 0; j < 8; j++) x[j] = (&raw[j * NV / 4].x)[j * NV % 4 + d];
         split_pieces(x, p);
         // Rows of four dims, 64 bytes, would meet in the same banks for
         // threads two apart: the row's place is turned by bits 3, 4 of the dim.
-        const int slot = 4 * vd + (d ^ ((vd >> 1) & 3));
+        const int dim = NV * vd + d, slot = dim ^ ((dim >> 3) & 3);
 #pragma unroll
         for (int i = 0; i < 3; i++)
           *(uint4*)(Vp + (i * (KT / 8) + vg) * T::VS + slot * 16) = p[i];
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
+      for (int j = 0; j < NV; j++) {
         const int u = j * 128 + su, key = u / (HD / 8), g = u % (HD / 8);
-        const float x[8] = {raw[2 * j].x,     raw[2 * j].y,     raw[2 * j].z,     raw[2 * j].w,
-                            raw[2 * j + 1].x, raw[2 * j + 1].y, raw[2 * j + 1].z, raw[2 * j + 1].w};
+        const float4 a = raw[2 * j], b = raw[2 * j + 1];
+        const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
         split_pieces(x, p);
 #pragma unroll
         for (int i = 0; i < 3; i++)
@@ -1398,15 +1411,15 @@ void launch_combine_rows(const float* ws, const float* gate, float* out, int64_t
 }
 
 // How the prefill attention deals its keys to workgroups: `splits` runs of
-// tps tiles each (1: the whole range, no workspace), and whether the combine
-// can also write the fp6 panel of the output.
+// tps tiles of kt keys each (1: the whole range, no workspace), and whether
+// the combine can also write the fp6 panel of the output.
 struct PrefillSplit {
-  int splits, tps;
+  int splits, tps, kt;
   bool panel;
 };
 
 PrefillSplit prefill_split(int64_t position, int64_t n, int64_t heads, int64_t hd, int64_t window,
-                           int gw, int kt) {
+                           int gw) {
   // Tiles of `keys` keys that a block of `queries` tokens walks.
   auto tiles_of = [&](int64_t b, int64_t queries, int64_t keys) {
     const int64_t first = b * queries, last = (first + queries < n ? first + queries : n) - 1;
@@ -1417,7 +1430,9 @@ PrefillSplit prefill_split(int64_t position, int64_t n, int64_t heads, int64_t h
   // Calls with 512 or more blocks of 64 (query, head) pairs, or fewer than 4
   // tiles of 32 keys, keep their keys whole and need no workspace. The panel
   // is offered where those blocks, brought to 512 by splitting runs of at
-  // least two such tiles, have at most 64 splits.
+  // least two such tiles, have at most 64 splits. The line does not follow the
+  // tiles below: it is the one by which callers know which calls may allocate
+  // and which write a panel.
   const int64_t q64 = 64 / gw, blocks64 = (n + q64 - 1) / q64;
   int64_t longest = 1;
   for (int64_t b = 0; b < blocks64; b++) longest = std::max(longest, tiles_of(b, q64, 32));
@@ -1429,6 +1444,11 @@ PrefillSplit prefill_split(int64_t position, int64_t n, int64_t heads, int64_t h
     splits32 = (longest + run - 1) / run;
     if (n * heads * splits32 * (hd + 4) * 4 > (1ll << 30) || splits32 > 4096) splits32 = 1;
   }
+  // hd 64: tiles of 64 keys, but of 32 where the longest range is one or three
+  // of those, half of whose last tile of 64 would be empty work (16 / 4 heads,
+  // tiles of 32 against 64, us: 32 tokens from 0 4.9 against 6.1, 96 from 0
+  // 8.1 against 9.2; two tiles of 32, 64 from 0: 6.5 against 6.2).
+  const int kt = hd == 128 || longest == 1 || longest == 3 ? 32 : 64;
   const int64_t qb = kPQ * (4 / gw), by = (n + qb - 1) / qb;
   int64_t tmax = 1, total = 0;
   for (int64_t b = 0; b < by; b++) {
@@ -1437,9 +1457,10 @@ PrefillSplit prefill_split(int64_t position, int64_t n, int64_t heads, int64_t h
     total += t;
   }
   total *= heads / gw;
-  if (splits32 == 1) return {1, (int)tmax, false};
+  if (splits32 == 1) return {1, (int)tmax, kt, false};
   // Runs of equal length that make about kTargetWorkgroups of them (two to a
-  // CU; 256, 384, 640 .. 1536 were slower or equal at 17 shapes), at most 64 to a row (the row combine's lanes) and 1 GiB of partials.
+  // CU; 256, 384, 640 .. 1536 were slower or equal at 17 shapes), at most 64
+  // to a row (the row combine's lanes) and 1 GiB of partials.
   constexpr int64_t kTargetWorkgroups = 512;
   int64_t tps = (total + kTargetWorkgroups - 1) / kTargetWorkgroups;
   tps = std::max(tps, (tmax + 63) / 64);
@@ -1449,16 +1470,16 @@ PrefillSplit prefill_split(int64_t position, int64_t n, int64_t heads, int64_t h
     tps *= 2;
     splits = (tmax + tps - 1) / tps;
   }
-  return {(int)splits, (int)tps, splits32 <= 64 && splits > 1};
+  return {(int)splits, (int)tps, kt, splits32 <= 64 && splits > 1};
 }
 
-template <int HD>
+template <int HD, int KT>
 void launch_prefill(int gw, dim3 grid, hipStream_t st, const float* q, const float* keys,
                     const float* values, const float* gate, float* out, float* ws, int position,
                     int n, int heads, int kv_dim, int group, int window, float scale, int splits,
                     int tps) {
-  auto k = gw == 4 ? attention_prefill_kernel<HD, 4>
-         : gw == 2 ? attention_prefill_kernel<HD, 2> : attention_prefill_kernel<HD, 1>;
+  auto k = gw == 4 ? attention_prefill_kernel<HD, 4, KT>
+         : gw == 2 ? attention_prefill_kernel<HD, 2, KT> : attention_prefill_kernel<HD, 1, KT>;
   hipLaunchKernelGGL(k, grid, dim3(kThreads), 0, st, q, keys, values, gate, out, ws, position, n,
                      heads, kv_dim, group, window, scale, splits, tps);
 }
@@ -1798,8 +1819,7 @@ static int attention_impl(const float* q, const float* keys, const float* values
       ((uintptr_t)out & 15) == 0) {
     const int64_t group = heads / kv_heads;
     const int gw = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
-    const int kt = hd == 128 ? PrefillTile<128>::KT : PrefillTile<64>::KT;
-    const PrefillSplit sp = prefill_split(position, n, heads, hd, window, gw, kt);
+    const PrefillSplit sp = prefill_split(position, n, heads, hd, window, gw);
     if (panel != nullptr && !sp.panel) return DNX_EINVAL;
     float* ws = nullptr;
     if (sp.splits > 1 && (ws = attention_workspace((size_t)n * heads * sp.splits * (hd + 4) * 4)) ==
@@ -1809,18 +1829,13 @@ static int attention_impl(const float* q, const float* keys, const float* values
     const int64_t qb = kPQ * (4 / gw);
     const dim3 grid((unsigned)(heads / gw), (unsigned)((n + qb - 1) / qb), (unsigned)sp.splits);
     const hipStream_t st = (hipStream_t)stream;
-    if (hd == 128) {
-      launch_prefill<128>(gw, grid, st, q, keys, values, gate, out, ws, (int)position, (int)n,
-                          (int)heads, (int)(kv_heads * hd), (int)group, (int)window, scale,
-                          sp.splits, sp.tps);
-    } else {
-      launch_prefill<64>(gw, grid, st, q, keys, values, gate, out, ws, (int)position, (int)n,
-                         (int)heads, (int)(kv_heads * hd), (int)group, (int)window, scale,
-                         sp.splits, sp.tps);
-    }
+    auto launch = hd == 128 ? launch_prefill<128, 32>
+                : sp.kt == 32 ? launch_prefill<64, 32> : launch_prefill<64, 64>;
+    launch(gw, grid, st, q, keys, values, gate, out, ws, (int)position, (int)n, (int)heads,
+           (int)(kv_heads * hd), (int)group, (int)window, scale, sp.splits, sp.tps);
     if (hipGetLastError() != hipSuccess) return DNX_ELAUNCH;
     if (sp.splits > 1) {
-      const RowSplits rsp{(int)position, (int)n, (int)window, (int)qb, kt, sp.tps};
+      const RowSplits rsp{(int)position, (int)n, (int)window, (int)qb, sp.kt, sp.tps};
       if (hd == 128) {
         launch_combine_rows<128>(ws, gate, out, heads, sp.splits, n * heads, panel, rsp, st);
       } else {

@@ -122,7 +122,9 @@ def test_attention(gpu_ready, orc, heads, kv, hd, pos, n, window, gated):
 # or 64 keys to a product step), of the window, and of the splits.
 @pytest.mark.parametrize("hd", [64, 128])
 @pytest.mark.parametrize("heads,kv,pos,n,window", [
-    (1, 1, 0, 8, 0), (4, 1, 23, 9, 0), (2, 1, 15, 16, 0), (2, 2, 16, 17, 0), (4, 1, 0, 65, 0),
+    (1, 1, 0, 8, 0), (4, 1, 0, 32, 0), (4, 1, 16, 17, 0), (8, 2, 31, 34, 0), (2, 2, 30, 66, 0),
+    (4, 1, 70, 27, 0), (2, 1, 60, 33, 32), (8, 2, 100, 18, 80), (32, 4, 269, 89, 0),
+    (4, 1, 23, 9, 0), (2, 1, 15, 16, 0), (2, 2, 16, 17, 0), (4, 1, 0, 65, 0),
     (8, 2, 62, 33, 1), (3, 1, 95, 31, 31), (4, 4, 97, 64, 32), (6, 3, 300, 40, 33),
     (8, 4, 511, 129, 64), (2, 1, 4095, 10, 0), (5, 5, 127, 128, 65)])
 def test_prefill_attention_edges(gpu_ready, orc, heads, kv, pos, n, window, hd):
@@ -202,6 +204,42 @@ def test_prefill_attention_precision(gpu_ready, heads, kv, hd, pos, n, bar):
     err = np.linalg.norm(got - want) / np.linalg.norm(want)
     print(f"{heads}/{kv} hd={hd} {n} after {pos}: {err:.2e}", flush=True)
     assert err < bar
+
+
+@pytest.mark.parametrize("hd,heads,kv,pos,n,other,share", [
+    (64, 16, 4, 0, 32, (0, 64), 0.9),     # one tile of 32 keys costs less than one of 64
+    (64, 16, 4, 0, 81, (0, 128), 1.0)])   # three of 32 less than two of 64
+def test_prefill_attention_short_calls_cost(gpu_ready, hd, heads, kv, pos, n, other,
+                                             share):
+    """Calls that cost as much as a longer one beside them, or more, while
+    every tile had 64 keys at hd 64."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+
+    def us(pos, n):
+        q = torch.randn(n, heads, hd, device="cuda", generator=g)
+        keys = torch.randn(pos + n, kv, hd, device="cuda", generator=g)
+        values = torch.randn(pos + n, kv, hd, device="cuda", generator=g)
+        out = torch.empty(n, heads, hd, device="cuda")
+        s, graph, best = torch.cuda.Stream(), torch.cuda.CUDAGraph(), 1e9
+        call = lambda: D.attention(q, keys, values, None, out, pos, n, heads, kv, hd)
+        with torch.cuda.stream(s):
+            call()
+        s.synchronize()
+        with torch.cuda.graph(graph, stream=s):
+            for _ in range(20):
+                call()
+        for _ in range(10):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            graph.replay()
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b) * 50)
+        return best
+
+    took, longer = us(pos, n), us(*other)
+    print(f"hd={hd} {n} after {pos}: {took:.2f} us, {other[1]} after {other[0]}: {longer:.2f}")
+    assert took < share * longer, (took, longer)
 
 
 def special_prefill(rng, heads, kv, hd, pos, n):
