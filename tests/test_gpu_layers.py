@@ -208,11 +208,13 @@ def test_prefill_attention_precision(gpu_ready, heads, kv, hd, pos, n, bar):
 
 @pytest.mark.parametrize("hd,heads,kv,pos,n,other,share", [
     (64, 16, 4, 0, 32, (0, 64), 0.9),     # one tile of 32 keys costs less than one of 64
-    (64, 16, 4, 0, 81, (0, 128), 1.0)])   # three of 32 less than two of 64
+    (64, 16, 4, 0, 81, (0, 128), 1.0),    # three of 32 less than two of 64
+    (64, 16, 4, 0, 65, (0, 80), 1.0)])    # a last block of one token no more than a whole one
 def test_prefill_attention_short_calls_cost(gpu_ready, hd, heads, kv, pos, n, other,
                                              share):
-    """Calls that cost as much as a longer one beside them, or more, while
-    every tile had 64 keys at hd 64."""
+    """Calls that cost more than a longer one beside them while every tile had
+    64 keys at hd 64, and while lanes past the last token left before the
+    divisions."""
     g = torch.Generator(device="cuda").manual_seed(1)
 
     def us(pos, n):
