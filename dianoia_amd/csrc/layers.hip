@@ -1467,6 +1467,11 @@ PrefillSplit prefill_split(int64_t position, int64_t n, int64_t heads, int64_t h
   constexpr int64_t kTargetWorkgroups = 512;
   int64_t tps = (total + kTargetWorkgroups - 1) / kTargetWorkgroups;
   tps = std::max(tps, (tmax + 63) / 64);
+  // A split a tile writes partials that cost more than they spread where they
+  // are large: two tiles a split above 9 MB (at 18 MB, 89 tokens after 269, 32
+  // / 4 heads, hd 128: 20.1 -> 14.6 us; at 12.3 and 16.9 MB 15.5 -> 14.3 and
+  // 17.7 -> 15.5; at 8.8 and 5.4 MB 11.8 -> 13.2 and 12.5 -> 13.3).
+  if (n * heads * tmax * (hd + 4) * 4 > 9000000) tps = std::max<int64_t>(tps, 2);
   if (tps >= tmax) tps = std::max<int64_t>(1, (tmax + 1) / 2);
   int64_t splits = (tmax + tps - 1) / tps;
   while (splits > 2 && n * heads * splits * (hd + 4) * 4 > (1ll << 30)) {

@@ -209,12 +209,13 @@ def test_prefill_attention_precision(gpu_ready, heads, kv, hd, pos, n, bar):
 @pytest.mark.parametrize("hd,heads,kv,pos,n,other,share", [
     (64, 16, 4, 0, 32, (0, 64), 0.9),     # one tile of 32 keys costs less than one of 64
     (64, 16, 4, 0, 81, (0, 128), 1.0),    # three of 32 less than two of 64
-    (64, 16, 4, 0, 65, (0, 80), 1.0)])    # a last block of one token no more than a whole one
+    (64, 16, 4, 0, 65, (0, 80), 1.0),     # a last block of one token no more than a whole one
+    (128, 32, 4, 269, 89, (400, 89), 1.0)])   # splits of two tiles no more than a longer range's
 def test_prefill_attention_short_calls_cost(gpu_ready, hd, heads, kv, pos, n, other,
                                              share):
     """Calls that cost more than a longer one beside them while every tile had
-    64 keys at hd 64, and while lanes past the last token left before the
-    divisions."""
+    64 keys at hd 64, while lanes past the last token left before the
+    divisions, and while large partials were split by the tile."""
     g = torch.Generator(device="cuda").manual_seed(1)
 
     def us(pos, n):
