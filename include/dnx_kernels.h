@@ -471,10 +471,10 @@ int dnx_short_conv(const float* bcx, const float* weight, float* history, float*
 // is exactly down to 2^-110 (2e-7 of it is lost at 2^-112, 2e-3 at 2^-125);
 // decode-shaped calls (fewer than 256 head-token pairs, more than 256 keys)
 // split the keys over workgroups.
-// Both may add a combine pass over a library-owned workspace grown on
-// demand: a first call at a larger shape allocates (not inside a graph
-// capture), and calls that overlap (other streams, other threads) must not
-// share the library. Otherwise at most dnx_attention_max_keys(hd) keys per
+// Both may add a combine pass over a library-owned workspace: the first call
+// on the matrix cores that splits its keys, and a first decode-shaped call at
+// a larger shape, allocate (not inside a graph capture), and calls that
+// overlap (other streams, other threads) must not share the library. Otherwise at most dnx_attention_max_keys(hd) keys per
 // token.
 int64_t dnx_attention_max_keys(int64_t hd);
 int dnx_attention(const float* q, const float* keys, const float* values, const float* gate,
