@@ -308,8 +308,7 @@ def test_prepacked_gemm_tile_edges(gpu_ready, q8, rows, cols, n):
 def test_prepacked_gemm_128_rows_many_stages(gpu_ready, orc, q8, rows, cols, n):
     """128-row tiles over 5 and 6 stages of K (Q8: 9 and 11), so that both weight
     buffers are filled again while the other is multiplied; K is not split.
-    Q4 gives the bits of the kernel on the engine's own layout; both stay
-    within the products' bar."""
+    Q4 gives the bits of the kernel on the engine's own layout."""
     rng = np.random.default_rng(rows + cols)
     qs, sc = (synth.q8_weights if q8 else synth.q4_weights)(rng, rows, cols)
     xs = synth.activations(rng, n, cols)
@@ -324,9 +323,16 @@ def test_prepacked_gemm_128_rows_many_stages(gpu_ready, orc, q8, rows, cols, n):
     if not q8:
         D.gemm_q4_f6(dev(qs), dev(sc), panel, y, rows, cols, n)
         assert np.array_equal(bits(got), bits(host(y).reshape(n, rows)))
-    ref = (orc.gemm_q8 if q8 else orc.gemm_q4)(qs, sc, xs, n, threads=8, mode=1)
-    ok, worst_rel, worst_abs = within_tolerance(got, ref)
-    assert ok, (worst_rel, worst_abs)
+    # Every eighth row against the exact products: 33 or 41 blocks, each with a
+    # scale product within 2^-22 and one float32 addition, so below 45 * 2^-24 =
+    # 2.7e-6 of the terms' magnitude; the products' bar is 1e-5. (Q8 outputs are
+    # about 30: a bar by element would be one on the values near zero.)
+    xq, xsc = orc.quantize_q8(xs)
+    qs, sc, got = qs[::8], sc[::8], got[:, ::8]
+    d = (orc.block_dots_q8 if q8 else orc.block_dots_q4)(qs, xq).astype(np.float64)
+    scale = sc if q8 else sc.view(np.float16).astype(np.float32)
+    terms = d * (scale[None] * xsc[:, None]).astype(np.float32)
+    assert np.max(np.abs(got - terms.sum(2)) / np.abs(terms).sum(2)) < 1e-5
 
 
 @pytest.mark.parametrize("kernel", ["f6", "f6p", "f6s", "i8p", "i8p_wide", "i8p_split"])
