@@ -478,9 +478,10 @@ swiglu_kernel(float* __restrict__ g, const float* __restrict__ u, int64_t count)
 // IEEE divisions, which took a third of the double operations, without
 // their scaling and special cases, none of which the operands need:
 //  - |v| / sqrt 2 as a product with the rounded reciprocal and one residual
-//    step, which rounds as the division does for every float (checked over
-//    all mantissas; the step does not depend on the exponent);
+//    step;
 //  - 1 / d for d in [1, 3.4] by Newton steps from the hardware's reciprocal.
+// The result is that of the two divisions for each of the 2^32 floats
+// (tests/test_gpu_glue.py goes through them all).
 // |v| above 10 counts as 10: there poly * exp(-x^2) is below 1e-22 and the
 // result 1 either way, and infinities and NaN need no case of their own (v
 // itself enters the last product).
