@@ -290,26 +290,26 @@ __global__ void __launch_bounds__(kThreads) gemm_float_kernel(FParams p) {
         for (int j = 0; j < 2; j++)
 #pragma unroll
           for (int v = 0; v < 16; v++) d[i][j][v] = 0.0f;
+      // The smallest pieces first: each MFMA rounds its sum, and only the last
+      // two then do so at its full size.
+      bf8 w[2][2];
 #pragma unroll
-      for (int h = 0; h < 2; h++) {
-        bf8 a[TM][3], w[2];
+      for (int h = 0; h < 2; h++)
 #pragma unroll
         for (int j = 0; j < 2; j++)
-          w[j] = __builtin_bit_cast(bf8, *(const uint4*)(bb + (2 * h + c) * T::kFB + j * 512));
+          w[h][j] = __builtin_bit_cast(bf8, *(const uint4*)(bb + (2 * h + c) * T::kFB + j * 512));
 #pragma unroll
-        for (int i = 0; i < TM; i++)
+      for (int pc = 2; pc >= 0; pc--)
 #pragma unroll
-          for (int pc = 0; pc < 3; pc++)
-            a[i][pc] = __builtin_bit_cast(
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+          for (int i = 0; i < TM; i++) {
+            const bf8 a = __builtin_bit_cast(
                 bf8, *(const uint4*)(ab + (pc * 4 + 2 * h + c) * T::kFA + i * 512));
 #pragma unroll
-        for (int pc = 0; pc < 3; pc++)
-#pragma unroll
-          for (int i = 0; i < TM; i++)
-#pragma unroll
             for (int j = 0; j < 2; j++)
-              d[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][pc], w[j], d[i][j], 0, 0, 0);
-      }
+              d[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, w[h][j], d[i][j], 0, 0, 0);
+          }
 #pragma unroll
       for (int j = 0; j < 2; j++) {
         const float sw =

@@ -105,6 +105,26 @@ def test_float_gemm_tile_edges(gpu_ready, fmt, rows, cols, n):
     assert np.array_equal(np.isnan(y[n // 2]), w == 0)
 
 
+@pytest.mark.parametrize("fmt,rows,cols,n,bar", [
+    ("q8", 514, 992, 179, 9.77e-8), ("q8", 1232, 1152, 11, 9.89e-8), ("q4", 973, 544, 69, 8.94e-8),
+    ("q4", 2949, 960, 19, 9.52e-8), ("q4", 1091, 1408, 26, 1.006e-7)])
+def test_float_gemm_precision(gpu_ready, fmt, rows, cols, n, bar):
+    """No further from 64 bits than with K in the shorter parts that four waves
+    of 32 tokens took, whose error on these inputs is the bar. (An output is
+    rounded B = cols / 32 times at its growing size, a random walk of sqrt(B /
+    2) roundings, and the blocks' own sums, the small pieces first, add 2 to
+    the B / 2: with 2^-24 / sqrt(12) each, 5.6e-8 at 544 columns and 8.4e-8 at
+    1408; measured 7.6e-8 and 9.2e-8.)"""
+    rng = np.random.default_rng(rows + cols + n)
+    qs, sc = (synth.q8_weights if fmt == "q8" else synth.q4_weights)(rng, rows, cols)
+    xs = rng.standard_normal((n, cols)).astype(np.float32)
+    y = gemm_float(fmt, qs, sc, xs, rows, cols, n)
+    exact, _ = exact_mode0(fmt, qs, sc, xs)
+    err = np.linalg.norm(y - exact) / np.linalg.norm(exact)
+    print(f"float gemm {fmt} {rows}x{cols} n={n}: {err:.3e}", flush=True)
+    assert err < bar
+
+
 def test_float_gemm_reference_gpu_test_shapes(gpu_ready, orc):
     """The reference's own GPU linear test (test/gpu_linear_test.dart:26-45):
     weights and inputs uniform in [-1, 1), within 1e-4 + 1e-5 |cpu| of CPU
