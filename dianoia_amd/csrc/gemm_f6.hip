@@ -1233,8 +1233,8 @@ int f6p_row_groups(int64_t rows, int64_t cols, int64_t n, bool q8) {
   const int per = f6_split_blocks((int)(tm * ((gn + 2) / 3)), B);
   const int64_t splits = (B + per - 1) / per;
   const double blocks = per < B ? per : B;
-  int best = 3;
-  double best_ns = 0.0;
+  int best = 0;
+  double best_ns = 1e30;
   for (int sn = 1; sn <= 4; sn++) {
     if (q8 && sn == 2) continue;
     const int64_t wgs = tm * ((gn + sn - 1) / sn) * splits;
@@ -1242,7 +1242,7 @@ int f6p_row_groups(int64_t rows, int64_t cols, int64_t n, bool q8) {
     const double block_ns = paired ? 240.0 : (q8 ? 80.0 : 48.0) * (sn + 1);
     const int64_t round = paired ? 512 : 256;
     const double ns = (double)((wgs + round - 1) / round) * (1000.0 + blocks * block_ns);
-    if (sn == 1 || ns < best_ns) {
+    if (ns < best_ns) {
       best = sn;
       best_ns = ns;
     }

@@ -81,7 +81,7 @@ DNX_DEV uint32_t bf16x2(int a, int b) {
 }
 
 // 8 weights of a block (k = 8c .. 8c + 7 of one K half) as one 16-byte bf16
-// fragment, from the block's integer values in w[0..31].
+// fragment, from their integer values in w[0..7].
 DNX_DEV uint4 weight_frag(const int* w) {
   return make_uint4(bf16x2(w[0], w[1]), bf16x2(w[2], w[3]), bf16x2(w[4], w[5]),
                     bf16x2(w[6], w[7]));
@@ -472,8 +472,6 @@ FloatCost float_cost(int64_t rows, int64_t cols, int64_t n, double round_us, dou
     if (want > B || (want > 1 && !may_split)) break;
     const int64_t run = ((B + want - 1) / want + T::PAR - 1) / T::PAR * T::PAR;
     const int64_t splits = (B + run - 1) / run;
-    // Partials of more than 1 GiB are not worth their memory.
-    if (splits > 1 && splits * n * rows > (1ll << 28)) break;
     const double rounds = (double)((tiles * splits + 255) / 256);
     const double us = rounds * (round_us + stage_us * (double)(run / T::PAR)) +
                       (splits > 1 ? 1.8 + 1.5e-6 * (double)(splits * n * rows) : 0.0);
