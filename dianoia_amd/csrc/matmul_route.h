@@ -18,11 +18,20 @@ enum class MatmulStep { kGemvFloat, kGemmFloat, kGemv, kQuantize, kGemm, kQuanti
 
 inline int64_t align256(int64_t v) { return (v + 255) & ~(int64_t)255; }
 
-// The fp6-MFMA GEMM wins over quantize + int8-MFMA GEMM only at large
-// prefill shapes: its 128-token x 96-row tiles and 16-block stages cost a
-// fixed ~5 us more (measured, graph-timed: at 768-2304 rows it loses at every
-// n <= 512; at 6144 x 2048 it wins from about 375 tokens: 26.0 against 29.6 us,
-// 512 tokens 29.2 against 32.6 us).
+// The fp6-MFMA GEMM against quantize + int8-MFMA GEMM (us with the quantizer,
+// graph-timed, six weight copies in turn). On the engine's layout (96-row
+// tiles): 6144 x 2048 at 256 / 320 / 375 / 512 / 1024 tokens 25.3 / 23.0 / 23.3
+// / 26.1 / 46.0 against 24.0 / 25.2 / 30.4 / 31.8 / 58.2, 4096 x 4096 at 320 /
+// 512 37.6 / 38.7 against 37.7 / 51.0; 4096 x 1024 at 320 / 512 ties (15.2 /
+// 15.7 against 15.0 / 15.3), and with fewer rows it loses up to 512 tokens
+// (3072 x 1024 at 375 / 512 19.2 / 21.6 against 15.4 / 15.1, 2048 x 2048 at 320
+// / 512 20.7 / 21.8 against 19.5 / 21.6). On prepacked weights (dnx_gemm_q4_f6p,
+// 32 to 128 rows) against the chunk route below: 6144 x 2048 at 256 / 320 / 512
+// 23.7 / 20.4 / 23.6 against 20.7 / 22.0 / 30.9, 2048 x 2048 at 512 19.7
+// against 14.7. The line is one for both, and leaves two ranges to the int8
+// GEMM where the prepacked kernel is the faster by now: above 512 tokens with
+// fewer rows (2048 x 2048 at 1024 21.8 against 26.6, 3072 x 1024 at 640 13.4
+// against 15.5) or K above 4096 (2048 x 6144 at 1000 43.0 against 70.9).
 inline bool matmul_uses_f6(bool q4, int64_t rows, int64_t cols, int64_t n) {
   return q4 && n >= 320 && rows >= 4096 && cols <= 4096;
 }
@@ -33,10 +42,13 @@ inline bool matmul_uses_f6(bool q4, int64_t rows, int64_t cols, int64_t n) {
 // 375 frames, the callers' 128 and 256): with a prepacked copy of the
 // weights (the lab_gpu_* command buffer keeps one per weight region) it runs
 // as the f6 panel quantizer + dnx_gemm_q4_f6s, one launch over the whole K.
-// Measured against quantize + int8 GEMM (graph-timed): 6144 x 2048 at 8..64
-// tokens 7.5-9.4 against 11.0-15.1 us, at 128 / 256 tokens 14.7 / 20.7
-// against 18.1 / 23.0; the audio shapes at 375 tokens 8.1-16.4 against
-// 11.7-19.2.
+// Measured against quantize + int8 GEMM (skinny, chunk or tile kernel by
+// shape; us, graph-timed with the quantizer): 6144 x 2048 at 8 / 16 / 32 / 64
+// tokens 8.0 / 8.1 / 8.5 / 10.3 against 11.7 / 12.9 / 13.0 / 15.6, at 128 / 256
+// 12.8 / 20.7 against 18.9 / 24.0; 3072 x 1024 at 64 / 512 6.5 / 14.8 against
+// 8.1 / 15.1; 2048 x 2048 at 33 / 64 / 128 7.9 / 8.0 / 8.6 against 10.6 / 11.8 /
+// 12.1; 512 x 2048, 2048 x 512, 4096 x 1024 and 1024 x 4096 at 375 9.7 / 8.7 /
+// 14.4 / 17.0 against 12.7 / 13.4 / 15.0 / 20.5.
 inline bool matmul_uses_f6_chunk(bool q4, int64_t rows, int64_t cols, int64_t n) {
   return q4 && n >= 5 && n <= 512 && !matmul_uses_f6(q4, rows, cols, n);
 }
@@ -45,16 +57,17 @@ inline bool matmul_uses_f6_chunk(bool q4, int64_t rows, int64_t cols, int64_t n)
 // projector at its 1024 patches, lib/src/vision_encoder.dart:252-316) with
 // a prepacked copy of the weights (the lab_gpu_* command buffer keeps one
 // per weight region): the int8 panel quantizer + dnx_gemm_q8_i8p.
-// Measured against quantize + int8 GEMM (graph-timed, weights rotated past
-// the MALL): 1152 x 4320 and 4320 x 1152 at 1024 tokens 32.0-33.1 /
-// 26.3-27.1 against 41.9-42.6 / 29.3-30.1 us, 4096 x 4096 at 1024 tokens
-// 53.1-53.7 against 78.3-84.7, 1152 x 1152 at 1024 tokens 14.5 against
-// 17.3, 1024 x 1024 at 256 / 512 / 1024 tokens 11.6 / 13.9 / 13.0-13.9
-// against 12.5 / 14.6 / 14.4-14.9, 768 x 768 at 512 tokens 12.3 against
-// 13.6. Below 256 tokens or 2^28 multiply-adds the int8 GEMM's smaller
-// tiles win or tie (1024 x 1024 and 2048 x 2048 at 128 tokens: 10.2 / 14.0
-// against 10.0 / 13.4); one shape inside the bounds measured slower (4096
-// x 1024 at 256 tokens, K of 32 blocks: 13.8 against 12.8).
+// Measured against quantize + int8 GEMM (us with the quantizer, graph-timed,
+// six weight copies in turn): 1152 x 4320 and 4320 x 1152 at 1024 tokens 33.6 /
+// 27.3 against 43.8 / 31.1, 4096 x 4096 at 1024 54.6 against 78.9, 1152 x 1152
+// at 1024 15.0 against 17.5, 1024 x 1024 at 1024 13.6 against 14.7, 6144 x 2048
+// at 256 18.2 against 24.3, 4096 x 1024 at 256 / 512 13.3 / 14.9 against 13.3 /
+// 15.6. Below 256 tokens the int8 GEMM wins (2048 x 2048 and 1024 x 1024 at 128
+// 10.9 / 7.4 against 13.9 / 10.1). Inside the bounds it has become the faster
+// where its chunk kernel takes the shape (1024 x 1024 at 256 / 512 7.7 / 10.0
+// against 12.1 / 14.3, 768 x 768 at 512 9.2 against 12.4, 2048 x 1024 at 256 9.4
+// against 12.6) and on 2048 x 2048 at 256 (14.5 against 15.7); the bounds are
+// older than that kernel and do not leave those shapes to it.
 inline bool matmul_uses_i8p(bool q4, int64_t rows, int64_t cols, int64_t n) {
   return !q4 && n >= 256 && rows * cols * n >= (1ll << 28);
 }
