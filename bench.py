@@ -652,8 +652,8 @@ def bench_layers(torch, D, timer, steps):
     decode over a 4096-position cache (32 query heads, 8 KV heads, hd 128;
     HBM-bound on the cached keys and values), RMSNorm over a 4096 x 2048
     prefill block, causal prefill attention of 512 tokens (same heads;
-    fp32 operands as three bf16 pieces, its rate beside the fp32 matrix
-    cores' peak) and the short convolution at 1 and 512 tokens.
+    fp32 operands as three bf16 pieces, its rate beside a sixth of the bf16
+    matrix cores' peak) and the short convolution at 1 and 512 tokens.
     Inputs generated on the GPU."""
     gen = torch.Generator(device="cuda").manual_seed(6)
     heads, kv, hd, pos = 32, 8, 128, 4095
@@ -705,7 +705,8 @@ def bench_layers(torch, D, timer, steps):
             "rms_norm_4096x2048_gbps": norm_bytes / means[1] / 1e6,
             "attention_prefill_512_ms": means[2],
             "attention_prefill_512_tflops": pre_flops / means[2] / 1e9,
-            "attention_prefill_512_frac_fp32_mfma": pre_flops / means[2] / 1e9 / 157.3,
+            # Six bf16 products for each float32 one.
+            "attention_prefill_512_frac_bf16_pieces": pre_flops / means[2] / 1e9 / (2500.0 / 6),
             "short_conv_2048x3_decode_ms": means[3],
             "short_conv_2048x3_prefill_512_ms": means[4],
             "short_conv_2048x3_prefill_512_gbps": conv_bytes / means[4] / 1e6,
@@ -1156,7 +1157,7 @@ MFMA_KERNELS = {
                               2 * 1024 * 4304 * 1152, I8_PEAK_TOPS),
     "gemm_float_kernel<false": ("c4 fc1 float inputs M=1024 (bf16)",
                                 2 * 1024 * 4320 * 1152, 2500.0),
-    "attention_prefill_kernel<128, 4>": ("prefill attention 512 tokens, 32/8 heads, hd 128",
+    "attention_prefill_kernel<128, 4, 32>": ("prefill attention 512 tokens, 32/8 heads, hd 128",
                                          4 * 128 * 32 * (512 * 513 // 2), 2500.0 / 6),
 }
 MFMA_COUNTERS = ("SQ_INSTS_MFMA", "SQ_VALU_MFMA_BUSY_CYCLES", "SQ_INSTS_VALU", "SQ_INSTS_LDS",
