@@ -947,11 +947,11 @@ DNX_DEV void mfma_pieces(const uint4* a, const uint4* b, v4f& big, v4f& low) {
 // One wave alone walks its keys, so a step's latency is what it costs: 32
 // keys a step in two chains, the next step's keys and this step's values
 // requested before the scores are formed (1000 tokens after 1000, 16 / 8
-// heads, hd 128, us; the finite call takes 110: one infinity among the values
-// 196, 236 with 16 keys a step and nothing ahead, and 4270 as a query at a time
-// in plain loads; every value infinite 369, 424 and 7060; a NaN among the keys
-// 107 to 138, every operand NaN 108 to 120. The float32 matrix cores alone,
-// with the keys shared in LDS, took 170 to 180 whatever the values).
+// heads, hd 128, us; the finite call takes 116: one infinity among the values
+// 202, 236 with 16 keys a step and nothing ahead, and 4270 as a query at a time
+// in plain loads; every value infinite 371, 424 and 7060; a NaN among the keys
+// 115 to 145, every operand NaN 124. The float32 matrix cores alone, with the
+// keys shared in LDS, took 170 to 180 whatever the values).
 template <int HD>
 DNX_DEV void prefill_special(const float* qp, const float* keys, const float* values, int kv_dim,
                              float sl, int k_lo, int k_hi, uint32_t see_lo, uint32_t see_n,
