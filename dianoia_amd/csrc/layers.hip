@@ -837,16 +837,16 @@ attention_combine_kernel(const float* __restrict__ ws, const float* __restrict__
 // multiply-add, one rounding before it.
 //
 // What bounds it: at prompt chunks the latency of one pass (launch, first
-// loads, splitting, two barriers: about 8 us with one tile, 1.8 us for each
-// more), at long prompts the MFMAs (six times the product's 2 flops, 215 of
-// 400 us at the 1.6 PFLOP/s a large bf16 product reaches) and the splitting
+// loads, splitting, two barriers: at hd 128 6.6 us with one tile, 2.3 us for
+// each more), at long prompts the MFMAs (six times the product's 2 flops, 215
+// of 400 us at the 1.6 PFLOP/s a large bf16 product reaches) and the splitting
 // and softmax they do not cover. Measured with the combine (us, graph-timed,
 // against the float32 MFMAs; heads / KV heads, hd): 64 tokens after 256,
-// 16 / 8, 128: 14.7 -> 11.9; 37 after 500, 8 / 8, 64: 11.3 -> 8.2; 512 from
-// 0, 32 / 8, 128: 42.7 -> 33.7; 1000 after 1000, 16 / 8, 128: 169 -> 98;
-// 1024 after 4000, 8 / 4, 64: 122 -> 80. 32 queries a wave (32x32x16 MFMAs,
+// 16 / 8, 128: 15.0 -> 12.2; 37 after 500, 8 / 8, 64: 11.6 -> 8.6; 512 from
+// 0, 32 / 8, 128: 41.7 -> 33.6; 1000 after 1000, 16 / 8, 128: 170 -> 99;
+// 1024 after 4000, 8 / 4, 64: 119 -> 78. 32 queries a wave (32x32x16 MFMAs,
 // half the LDS reads) gained 8% on the longest but needed 256 registers, and
-// took 13.2 us where this takes 9.1 for one tile.
+// was 4 us slower with one tile.
 constexpr int kPQ = 16;   // queries per wave
 
 typedef float v4f __attribute__((ext_vector_type(4)));
